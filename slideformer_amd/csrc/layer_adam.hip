@@ -183,6 +183,7 @@ struct StepArgs {
     uint64_t nvec;       // aligned groups of 4, starting at `head`
     uint64_t tail_start; // n - n % 16: first element of the reference's scalar tail
     Coeffs k;
+    bool misphased;      // no head aligns every stream: the kernels' misphased form
 };
 
 // One wave's run of 64 aligned groups (256 elements) of every stream, run w of
@@ -191,24 +192,40 @@ struct StepArgs {
 // and whose size covers only the run's valid groups, so the lanes of a partial
 // last run need no branch: their loads return 0 and their stores are dropped
 // by the hardware range check.
-template <typename TP, typename TG, typename TS>
+//
+// MIS is the form for streams that no head aligns together (moments that are
+// slices of a flat buffer beside parameters of their own, a rank's odd slice
+// of the grads): WaveIoU's accesses, and the lanes beyond a partial last run
+// leave first.  It is bound by HBM like the aligned form, since the hardware
+// splits a wave's misaligned access only at the run's two ends.  Measured on
+// MI355X, ms per launch at 39 M elements, one element per lane with scalar
+// accesses / this form / all streams aligned: (f32, bf16, f32) 0.317 / 0.165 /
+// 0.165, (bf16, bf16, f32) 0.321 / 0.157, (bf16, bf16, bf16) 0.284 / 0.104 /
+// 0.097.  It is kept beside the aligned form for those last few percent and
+// for the aligned form's written-through 16-bit stores.
+template <typename TP, typename TG, typename TS, bool MIS>
 __device__ __forceinline__ void update_run(const StepArgs& a, uint64_t w, uint32_t lane, bool has_coef, float coef)
 {
+    using IoP = std::conditional_t<MIS, WaveIoU<TP>, WaveIo<TP>>;
+    using IoG = std::conditional_t<MIS, WaveIoU<TG>, WaveIo<TG>>;
+    using IoS = std::conditional_t<MIS, WaveIoU<TS>, WaveIo<TS>>;
+    using IoO = std::conditional_t<MIS, WaveIoU<bf16_t>, WaveIo<bf16_t>>;
     const uint64_t left = a.nvec - w * 64;
     const uint32_t nel = (left < 64 ? static_cast<uint32_t>(left) : 64u) * kVec;
     const uint64_t e0 = a.head + w * 64 * kVec;
-    const rsrc_t rg = WaveIo<TG>::rsrc(a.g, e0, nel);
-    const rsrc_t rp = WaveIo<TP>::rsrc(a.p, e0, nel);
-    const rsrc_t rm = WaveIo<TS>::rsrc(a.m, e0, nel);
-    const rsrc_t rv = WaveIo<TS>::rsrc(a.v, e0, nel);
+    if (MIS && lane * kVec >= nel) return;
+    const auto rg = IoG::rsrc(a.g, e0, nel);
+    const auto rp = IoP::rsrc(a.p, e0, nel);
+    const auto rm = IoS::rsrc(a.m, e0, nel);
+    const auto rv = IoS::rsrc(a.v, e0, nel);
     float p[kVec], g[kVec], m[kVec], v[kVec];
 #if LA_SETPRIO
     __builtin_amdgcn_s_setprio(3);
 #endif
-    WaveIo<TG>::load4(rg, lane, g);
-    WaveIo<TP>::load4(rp, lane, p);
-    WaveIo<TS>::load4(rm, lane, m);
-    WaveIo<TS>::load4(rv, lane, v);
+    IoG::load4(rg, lane, g);
+    IoP::load4(rp, lane, p);
+    IoS::load4(rm, lane, m);
+    IoS::load4(rv, lane, v);
 #if LA_SETPRIO
     __builtin_amdgcn_s_setprio(0);
 #endif
@@ -217,10 +234,10 @@ __device__ __forceinline__ void update_run(const StepArgs& a, uint64_t w, uint32
         const float gj = has_coef ? g[j] * coef : g[j];
         adam_body(p[j], gj, m[j], v[j], a.k);
     }
-    WaveIo<TP>::store4(rp, lane, p);
-    WaveIo<TS>::store4(rm, lane, m);
-    WaveIo<TS>::store4(rv, lane, v);
-    if (a.out) WaveIo<bf16_t>::store4(WaveIo<bf16_t>::rsrc(a.out, e0, nel), lane, p);
+    IoP::store4(rp, lane, p);
+    IoS::store4(rm, lane, m);
+    IoS::store4(rv, lane, v);
+    if (a.out) IoO::store4(IoO::rsrc(a.out, e0, nel), lane, p);
 }
 
 // One element outside the aligned groups; the reference's scalar tail from
@@ -241,7 +258,7 @@ __device__ __forceinline__ void update_one(const StepArgs& a, uint64_t e, bool h
     if (a.out) a.out[e] = static_cast<uint16_t>(f32_to_bf16_bits(p));
 }
 
-template <typename TP, typename TG, typename TS>
+template <typename TP, typename TG, typename TS, bool MIS>
 __global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
 {
     const bool has_coef = a.coef != nullptr;
@@ -254,7 +271,7 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t nwaves = stride >> 6;
     for (uint64_t w = wave_uniform(tid >> 6); w * 64 < a.nvec; w += nwaves)
-        update_run<TP, TG, TS>(a, w, lane, has_coef, coef);
+        update_run<TP, TG, TS, MIS>(a, w, lane, has_coef, coef);
 
     // Elements outside the aligned groups: [0, head) and [head + 4*nvec, n).
     const uint64_t vec_end = a.head + a.nvec * kVec;
@@ -274,7 +291,9 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
 // arguments count 8-element groups here.
 constexpr int kVec16 = 8;
 
-template <typename Conv> struct WaveIo16x8 {
+template <typename Conv, bool MIS> struct WaveIo16x8;
+
+template <typename Conv> struct WaveIo16x8<Conv, false> {
     __device__ __forceinline__ static rsrc_t rsrc(const void* base, uint64_t e0, uint32_t nel)
     {
         return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(static_cast<const uint16_t*>(base) + e0), 0,
@@ -299,22 +318,48 @@ template <typename Conv> struct WaveIo16x8 {
                                                kAuxSt);
     }
 };
+// Streams that disagree in alignment phase, as WaveIoU16.
+template <typename Conv> struct WaveIo16x8<Conv, true> {
+    __device__ __forceinline__ static uint16_t* rsrc(const void* base, uint64_t e0, uint32_t)
+    {
+        return const_cast<uint16_t*>(static_cast<const uint16_t*>(base) + e0);
+    }
+    __device__ __forceinline__ static void load8(const uint16_t* r, uint32_t lane, float (&x)[kVec16])
+    {
+        const u32x4 u = vload<u32x4_a2>(r + lane * kVec16);
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            x[2 * k] = Conv::to_f32(w[k] & 0xffffu);
+            x[2 * k + 1] = Conv::to_f32(w[k] >> 16);
+        }
+    }
+    __device__ __forceinline__ static void store8(uint16_t* r, uint32_t lane, const float (&x)[kVec16])
+    {
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) w[k] = Conv::from_f32x2(x[2 * k], x[2 * k + 1]);
+        vstore<u32x4_a2>(r + lane * kVec16, u32x4{w[0], w[1], w[2], w[3]});
+    }
+};
 template <typename T> struct Conv16;
 template <> struct Conv16<bf16_t> { using type = ConvBf16; };
 template <> struct Conv16<f16_t> { using type = ConvF16; };
 
-template <typename T16, typename TG16>
+template <typename T16, typename TG16, bool MIS>
 __device__ __forceinline__ void update_run16(const StepArgs& a, uint64_t w, uint32_t lane, bool has_coef, float coef)
 {
-    using IoS = WaveIo16x8<typename Conv16<T16>::type>;
-    using IoG = WaveIo16x8<typename Conv16<TG16>::type>;
+    using IoS = WaveIo16x8<typename Conv16<T16>::type, MIS>;
+    using IoG = WaveIo16x8<typename Conv16<TG16>::type, MIS>;
+    using IoO = WaveIo16x8<ConvBf16, MIS>;
     const uint64_t left = a.nvec - w * 64;
     const uint32_t nel = (left < 64 ? static_cast<uint32_t>(left) : 64u) * kVec16;
     const uint64_t e0 = a.head + w * 64 * kVec16;
-    const rsrc_t rg = IoG::rsrc(a.g, e0, nel);
-    const rsrc_t rp = IoS::rsrc(a.p, e0, nel);
-    const rsrc_t rm = IoS::rsrc(a.m, e0, nel);
-    const rsrc_t rv = IoS::rsrc(a.v, e0, nel);
+    if (MIS && lane * kVec16 >= nel) return;
+    const auto rg = IoG::rsrc(a.g, e0, nel);
+    const auto rp = IoS::rsrc(a.p, e0, nel);
+    const auto rm = IoS::rsrc(a.m, e0, nel);
+    const auto rv = IoS::rsrc(a.v, e0, nel);
     float p[kVec16], g[kVec16], m[kVec16], v[kVec16];
 #if LA_SETPRIO
     __builtin_amdgcn_s_setprio(3);
@@ -334,10 +379,10 @@ __device__ __forceinline__ void update_run16(const StepArgs& a, uint64_t w, uint
     IoS::store8(rp, lane, p);
     IoS::store8(rm, lane, m);
     IoS::store8(rv, lane, v);
-    if (a.out) WaveIo16x8<ConvBf16>::store8(WaveIo16x8<ConvBf16>::rsrc(a.out, e0, nel), lane, p);
+    if (a.out) IoO::store8(IoO::rsrc(a.out, e0, nel), lane, p);
 }
 
-template <typename TP, typename TG, typename TS>
+template <typename TP, typename TG, typename TS, bool MIS>
 __global__ __launch_bounds__(LA_BLOCK) void la_adamw16_kernel(StepArgs a)
 {
     static_assert(std::is_same<TP, TS>::value && std::is_same<TP, TG>::value, "all-16-bit triples only");
@@ -348,7 +393,7 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw16_kernel(StepArgs a)
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t nwaves = stride >> 6;
     for (uint64_t w = wave_uniform(tid >> 6); w * 64 < a.nvec; w += nwaves)
-        update_run16<TP, TG>(a, w, lane, has_coef, coef);
+        update_run16<TP, TG, MIS>(a, w, lane, has_coef, coef);
     const uint64_t vec_end = a.head + a.nvec * kVec16;
     const uint64_t nscalar = a.head + (a.n - vec_end);
     for (uint64_t s = tid; s < nscalar; s += stride) {
@@ -364,7 +409,6 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw16_kernel(StepArgs a)
 // its at most 21 elements outside the aligned groups.  Segments must not
 // overlap in memory.
 constexpr int kMaxSegs = 16;
-constexpr uint64_t kMaxSegScalars = 64;  // one wave's lanes
 // Segments of any size go in a batch: with the wave index and the segment
 // arguments in scalar registers, a Llama-3.1-8B layer's nine tensors (16-58 Mi
 // elements) batched run 1.1-1.7 % faster than separate launches of the big
@@ -383,7 +427,7 @@ struct MultiArgs {
     StepArgs seg[kMaxSegs];
 };
 
-template <typename TP, typename TG, typename TS>
+template <typename TP, typename TG, typename TS, bool MIS>
 __global__ __launch_bounds__(LA_BLOCK) void la_adamw_multi_kernel(MultiArgs a)
 {
     const bool has_coef = a.coef != nullptr;
@@ -394,7 +438,7 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw_multi_kernel(MultiArgs a)
     if (w < runs) {
         uint32_t s = 0;
         while (w >= a.run_begin[s + 1]) ++s;
-        update_run<TP, TG, TS>(a.seg[s], w - a.run_begin[s], lane, has_coef, coef);
+        update_run<TP, TG, TS, MIS>(a.seg[s], w - a.run_begin[s], lane, has_coef, coef);
         return;
     }
     const uint64_t s = w - runs;
@@ -607,6 +651,27 @@ int common_head(const uintptr_t* addr, const int* bytes, int count, int vec = kV
     return -1;
 }
 
+// The head of a call whose streams disagree in phase, for the misphased form: the h in [0, vec) that
+// leaves the fewest bytes per element in misaligned accesses (p, m and v are
+// read and written, g is only read, the bf16 copy only written).
+int best_head(const uintptr_t* addr, const int* bytes, int count, int vec = kVec)
+{
+    int best = 0, best_cost = INT32_MAX;
+    for (int h = 0; h < vec; ++h) {
+        int cost = 0;
+        for (int i = 0; i < count; ++i) {
+            const uintptr_t align = static_cast<uintptr_t>(vec * bytes[i]);
+            const bool twice = i == 0 || i == 2 || i == 3;
+            if ((addr[i] + static_cast<uintptr_t>(h) * bytes[i]) % align) cost += bytes[i] * (twice ? 2 : 1);
+        }
+        if (cost < best_cost) {
+            best_cost = cost;
+            best = h;
+        }
+    }
+    return best;
+}
+
 uint32_t grid_for(uint64_t work, uint64_t block, uint64_t cap)
 {
     uint64_t blocks = (work + block - 1) / block;
@@ -703,14 +768,15 @@ template <typename TP, typename TG, typename TS> int launch4(const StepArgs& a, 
     // lanes needed: every wave takes one run of 64 groups
     const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
     const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
-    return launch(la_adamw_kernel<TP, TG, TS>, dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
+    return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true> : la_adamw_kernel<TP, TG, TS, false>,
+                  dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
                   update_lds_bytes<TP, TG, TS>(), stream, a);
 }
 
 // The all-16-bit path: the call's groups are re-laid out as 8-element groups.
-// Pointers that share a 4-element phase but not an 8-element one (16-byte
-// alignment) keep the 4-element layout of la_adamw_kernel rather than the
-// all-scalar path.
+// Pointers that share a 4-element phase but not an 8-element one take the
+// misphased 8-element form too: 0.104 ms against 0.113 ms in the aligned
+// 4-element layout, (bf16, bf16, bf16) at 39 M elements.
 template <typename T> int launch16(const StepArgs& a4, hipStream_t stream)
 {
     StepArgs a = a4;
@@ -718,9 +784,10 @@ template <typename T> int launch16(const StepArgs& a4, hipStream_t stream)
                                reinterpret_cast<uintptr_t>(a.m), reinterpret_cast<uintptr_t>(a.v),
                                reinterpret_cast<uintptr_t>(a.out)};
     const int bytes[5] = {2, 2, 2, 2, 2};
-    const int h = common_head(addr, bytes, a.out ? 5 : 4, kVec16);
-    if (h < 0 || static_cast<uint64_t>(h) >= a.tail_start) {
-        if (a4.nvec > 0) return launch4<T, T, T>(a4, stream);
+    int h = common_head(addr, bytes, a.out ? 5 : 4, kVec16);
+    a.misphased = h < 0;
+    if (h < 0) h = best_head(addr, bytes, a.out ? 5 : 4, kVec16);
+    if (static_cast<uint64_t>(h) >= a.tail_start) {
         a.head = 0;
         a.nvec = 0;
     } else {
@@ -730,7 +797,8 @@ template <typename T> int launch16(const StepArgs& a4, hipStream_t stream)
     const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * kVec16));
     const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
     const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
-    return launch(la_adamw16_kernel<T, T, T>, dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
+    return launch(a.misphased ? la_adamw16_kernel<T, T, T, true> : la_adamw16_kernel<T, T, T, false>,
+                  dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
                   update16_lds_bytes<T>(), stream, a);
 }
 
@@ -746,10 +814,11 @@ template <typename TP, typename TG, typename TS> struct StepLauncher {
 
 template <typename TP, typename TG, typename TS> struct MultiLauncher {
     // waves: runs of every segment + one scalar wave per segment
-    static int run(const MultiArgs& a, uint64_t waves, hipStream_t stream)
+    static int run(const MultiArgs& a, uint64_t waves, bool misphased, hipStream_t stream)
     {
-        return launch(la_adamw_multi_kernel<TP, TG, TS>, dim3(static_cast<uint32_t>(waves * 64 / LA_BLOCK)),
-                      dim3(LA_BLOCK), multi_lds_bytes<TP, TG, TS>(), stream, a);
+        return launch(misphased ? la_adamw_multi_kernel<TP, TG, TS, true> : la_adamw_multi_kernel<TP, TG, TS, false>,
+                      dim3(static_cast<uint32_t>(waves * 64 / LA_BLOCK)), dim3(LA_BLOCK),
+                      multi_lds_bytes<TP, TG, TS>(), stream, a);
     }
 };
 
@@ -799,8 +868,10 @@ int prepare_step(int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, 
     a.coef = clip_coef;
     a.n = n;
     a.tail_start = n - n % 16;
-    const int h = common_head(addr, bytes, count);
-    if (h < 0 || static_cast<uint64_t>(h) >= a.tail_start) {
+    int h = common_head(addr, bytes, count);
+    a.misphased = h < 0;
+    if (h < 0) h = best_head(addr, bytes, count);
+    if (static_cast<uint64_t>(h) >= a.tail_start) {
         a.head = 0;
         a.nvec = 0;
     } else {
@@ -1180,6 +1251,7 @@ try {
     std::memset(&batch, 0, sizeof(batch));
     batch.coef = clip_coef;
     uint64_t runs = 0;
+    bool misphased = false;
     auto flush = [&]() -> int {
         if (batch.count == 0) return LA_OK;
         // one wave per run and per segment: the grid must fit the dispatch packet
@@ -1187,20 +1259,20 @@ try {
         // kMaxSegs segments)
         if (runs + batch.count > static_cast<uint64_t>(LA_MAX_GRID)) return LA_EINVAL;
         batch.run_begin[batch.count] = runs;
-        const int rc = dispatch_triple<MultiLauncher>(p_dtype, g_dtype, s_dtype, batch, runs + batch.count, st);
+        const int rc = dispatch_triple<MultiLauncher>(p_dtype, g_dtype, s_dtype, batch, runs + batch.count,
+                                                      misphased, st);
         std::memset(&batch, 0, sizeof(batch));
         batch.coef = clip_coef;
         runs = 0;
+        misphased = false;
         return rc;
     };
     for (int k = 0; k < count; ++k) {
         const StepArgs& a = args[k];
         if (a.n == 0) continue;
         const uint64_t seg_runs = (a.nvec + 63) / 64;
-        const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * kVec));
-        if (nscalar > kMaxSegScalars || seg_runs > LA_MAX_GRID / 2) {
-            // pointers out of phase (all elements scalar), or more runs than one
-            // batch holds: its own launch, which grid-strides
+        if (seg_runs > LA_MAX_GRID / 2) {
+            // more runs than one batch holds: its own launch, which grid-strides
             const int rc = dispatch_triple<StepLauncher>(p_dtype, g_dtype, s_dtype, a, st);
             if (rc != LA_OK) return rc;
             continue;
@@ -1211,6 +1283,7 @@ try {
         }
         batch.run_begin[batch.count] = runs;
         batch.seg[batch.count] = a;
+        misphased |= a.misphased;
         batch.count++;
         runs += seg_runs;
     }

@@ -246,6 +246,41 @@ template <typename Conv> struct WaveIo16 {
 template <> struct WaveIo<bf16_t> : WaveIo16<ConvBf16> {};
 template <> struct WaveIo<f16_t> : WaveIo16<ConvF16> {};
 
+// The same accesses for a call whose streams disagree in alignment phase.
+// fp32 streams keep the buffer accesses, which need 4-byte alignment only.
+// 16-bit streams may start at an odd element: they use global accesses of
+// 2-byte alignment (the compiler's unaligned-access mode, the default on this
+// target).  Those have no range check, so the caller masks the lanes beyond
+// the run.
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+
+template <typename T> struct WaveIoU;
+template <> struct WaveIoU<float> : WaveIo<float> {};
+
+template <typename Conv> struct WaveIoU16 {
+    __device__ __forceinline__ static uint16_t* rsrc(const void* base, uint64_t e0, uint32_t)
+    {
+        return const_cast<uint16_t*>(static_cast<const uint16_t*>(base) + e0);
+    }
+    __device__ __forceinline__ static void load4(const uint16_t* r, uint32_t lane, float (&x)[kVec])
+    {
+        const u32x2 u = vload<u32x2_a2>(r + lane * kVec);
+        x[0] = Conv::to_f32(u.x & 0xffffu);
+        x[1] = Conv::to_f32(u.x >> 16);
+        x[2] = Conv::to_f32(u.y & 0xffffu);
+        x[3] = Conv::to_f32(u.y >> 16);
+    }
+    __device__ __forceinline__ static void store4(uint16_t* r, uint32_t lane, const float (&x)[kVec])
+    {
+        const uint32_t lo = Conv::from_f32x2(x[0], x[1]);
+        const uint32_t hi = Conv::from_f32x2(x[2], x[3]);
+        vstore<u32x2_a2>(r + lane * kVec, u32x2{lo, hi});
+    }
+};
+template <> struct WaveIoU<bf16_t> : WaveIoU16<ConvBf16> {};
+template <> struct WaveIoU<f16_t> : WaveIoU16<ConvF16> {};
+
 // The value of lane 0 of the wave, as a wave-uniform value.  The wave index is
 // the same in every lane, but the compiler cannot prove it from threadIdx.x;
 // without this it keeps the index in vector registers, builds the buffer

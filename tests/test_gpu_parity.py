@@ -199,8 +199,8 @@ def test_all_16bit_triples_every_head_phase(kind, offsets, hip_device):
     whose lanes own 8 consecutive elements: the head that aligns every stream,
     the bf16 copy included, to 8-element (16-byte) groups, the 512-element
     runs, the remainder and the reference's scalar tail.  Every head phase
-    0-7, phases that agree only modulo 4 (then the call takes la_adamw_kernel's
-    4-element layout), sizes around 8, 16, 512 and the tail, with the bf16 copy and a clip
+    0-7, phases that agree only modulo 4 (then the call takes the kernel's
+    misphased form), sizes around 8, 16, 512 and the tail, with the bf16 copy and a clip
     coefficient: every bit equals the oracle's."""
     op, og, om, ov, oo = offsets
     log(f"16-bit triple {kind} offsets {offsets}")
@@ -514,7 +514,7 @@ MULTI_SIZES = [1, 3, 15, 16, 17, 255, 256, 257, 4099, 100_003, 7, 64, 1000, 33, 
 def test_multi_update_equals_separate_calls(triple, mode, hip_device):
     """21 segments of awkward sizes: 19 small ones and a 4 Mi-element one (two
     batched launches of up to 16) and one whose params are out of phase with
-    its grads (launched on its own).  Some sit at odd
+    its grads.  Some sit at odd
     element offsets inside their buffers; a clip coefficient applies and every
     other segment writes a bf16 copy.  Bit-exact with the same 21
     la_adam_update calls, and every segment with the oracle replaying them."""
@@ -576,8 +576,8 @@ def test_multi_update_equals_separate_calls(triple, mode, hip_device):
 # launch paths the product build takes only at sizes beyond one GPU: the
 # small-grid test build (64 waves per update launch, 2 workgroups per norm
 # launch, so at most 32 runs per multi batch and an own grid-stride launch for
-# a segment of more runs, which the product build gives a segment whose
-# pointers agree in phase only above 2^33 elements) against the product build
+# a segment of more runs, which the product build gives a segment only above
+# 2^33 elements) against the product build
 # ---------------------------------------------------------------------------
 
 SMALL_GRID_SIZES = [7, 16, 64 * 256 * 3 + 5, 64 * 256 * 40 + 13, 1_000_003]
