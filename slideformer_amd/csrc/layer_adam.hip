@@ -113,11 +113,13 @@
 // (f16, f16, f32) 0.812 / 0.789 / 0.786 / 0.802 / 0.803 / 0.835 and every
 // other triple of this layout best at 13 KiB (12 waves).  A previous build,
 // with the wave index in vector registers, was best at 16 KiB for
-// (f32, f32, f32) and at 10 KiB for (f16, f16, f32).  The all-16-bit triples
-// normally run la_adamw16_kernel (own cap below); with LA_WIDE16=0 they take
-// this kernel, best there at 8 KiB (bf16) and 10 KiB (f16) on the previous
-// build.  LA_UPDATE_LDS_BYTES, when defined, overrides the table for every
-// triple.
+// (f32, f32, f32) and at 10 KiB for (f16, f16, f32).  The all-16-bit triples,
+// whose waves move twice the elements (C2 shape, ms per launch at 10, 11, 12,
+// 13, 14 KiB; 4 elements per lane at its own best cap before them):
+// (bf16, bf16, bf16) 0.571-0.574 / 0.549-0.553, 0.547-0.551, 0.546-0.550,
+// 0.550-0.553, 0.560-0.561; (f16, f16, f16) 0.539-0.541 / 0.534-0.536,
+// 0.532-0.534, 0.531, 0.524-0.525, 0.524-0.526.  Kept: 12 and 13 KiB.
+// LA_UPDATE_LDS_BYTES, when defined, overrides the table for every triple.
 #ifdef LA_UPDATE_LDS_BYTES
 #define LA_UPDATE_LDS_OVERRIDE 1
 #else
@@ -180,7 +182,7 @@ struct StepArgs {
     const float* coef;   // clip coefficient (device), may be null
     uint64_t n;
     uint64_t head;       // elements before the first aligned group
-    uint64_t nvec;       // aligned groups of 4, starting at `head`
+    uint64_t nvec;       // aligned groups of lane_elems, starting at `head`
     uint64_t tail_start; // n - n % 16: first element of the reference's scalar tail
     Coeffs k;
     bool misphased;      // no head aligns every stream: the kernels' misphased form
@@ -258,37 +260,12 @@ __device__ __forceinline__ void update_one(const StepArgs& a, uint64_t e, bool h
     if (a.out) a.out[e] = static_cast<uint16_t>(f32_to_bf16_bits(p));
 }
 
-template <typename TP, typename TG, typename TS, bool MIS>
-__global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
-{
-    const bool has_coef = a.coef != nullptr;
-    const float coef = has_coef ? *a.coef : 1.0f;
-    const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * LA_BLOCK + threadIdx.x;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_BLOCK;
-
-    // Wave w owns run w: groups [64w, 64w + 64), 256 lane-contiguous elements
-    // per stream.  The grid is one-shot unless n exceeds LA_MAX_GRID runs.
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nwaves = stride >> 6;
-    for (uint64_t w = wave_uniform(tid >> 6); w * 64 < a.nvec; w += nwaves)
-        update_run<TP, TG, TS, MIS>(a, w, lane, has_coef, coef);
-
-    // Elements outside the aligned groups: [0, head) and [head + 4*nvec, n).
-    const uint64_t vec_end = a.head + a.nvec * kVec;
-    const uint64_t nscalar = a.head + (a.n - vec_end);
-    for (uint64_t s = tid; s < nscalar; s += stride) {
-        const uint64_t e = s < a.head ? s : vec_end + (s - a.head);
-        update_one<TP, TG, TS>(a, e, has_coef, coef);
-    }
-}
-
 // All-16-bit triples ((bf16, bf16, bf16), (f16, f16, f16)): every stream, the
 // bf16 copy included, has 2-byte elements, so a lane owns 8 consecutive
 // elements and moves each stream with one 16-byte access; one wave
 // instruction covers 512 elements (1 KiB) of a stream, and a launch needs
-// half the waves of the 4-element layout.  The per-element arithmetic and the
-// scalar path are the same as la_adamw_kernel's.  `head` and `nvec` of the
-// arguments count 8-element groups here.
+// half the waves of the 4-element layout.  `head` and `nvec` of the arguments
+// count 8-element groups here.
 constexpr int kVec16 = 8;
 
 template <typename Conv, bool MIS> struct WaveIo16x8;
@@ -346,17 +323,16 @@ template <typename T> struct Conv16;
 template <> struct Conv16<bf16_t> { using type = ConvBf16; };
 template <> struct Conv16<f16_t> { using type = ConvF16; };
 
-template <typename T16, typename TG16, bool MIS>
+template <typename T16, bool MIS>
 __device__ __forceinline__ void update_run16(const StepArgs& a, uint64_t w, uint32_t lane, bool has_coef, float coef)
 {
     using IoS = WaveIo16x8<typename Conv16<T16>::type, MIS>;
-    using IoG = WaveIo16x8<typename Conv16<TG16>::type, MIS>;
     using IoO = WaveIo16x8<ConvBf16, MIS>;
     const uint64_t left = a.nvec - w * 64;
     const uint32_t nel = (left < 64 ? static_cast<uint32_t>(left) : 64u) * kVec16;
     const uint64_t e0 = a.head + w * 64 * kVec16;
     if (MIS && lane * kVec16 >= nel) return;
-    const auto rg = IoG::rsrc(a.g, e0, nel);
+    const auto rg = IoS::rsrc(a.g, e0, nel);
     const auto rp = IoS::rsrc(a.p, e0, nel);
     const auto rm = IoS::rsrc(a.m, e0, nel);
     const auto rv = IoS::rsrc(a.v, e0, nel);
@@ -364,7 +340,7 @@ __device__ __forceinline__ void update_run16(const StepArgs& a, uint64_t w, uint
 #if LA_SETPRIO
     __builtin_amdgcn_s_setprio(3);
 #endif
-    IoG::load8(rg, lane, g);
+    IoS::load8(rg, lane, g);
     IoS::load8(rp, lane, p);
     IoS::load8(rm, lane, m);
     IoS::load8(rv, lane, v);
@@ -382,19 +358,41 @@ __device__ __forceinline__ void update_run16(const StepArgs& a, uint64_t w, uint
     if (a.out) IoO::store8(IoO::rsrc(a.out, e0, nel), lane, p);
 }
 
-template <typename TP, typename TG, typename TS, bool MIS>
-__global__ __launch_bounds__(LA_BLOCK) void la_adamw16_kernel(StepArgs a)
+// Elements a lane owns, the group size of `head` and `nvec`.
+template <typename TP, typename TG, typename TS> constexpr int lane_elems()
 {
-    static_assert(std::is_same<TP, TS>::value && std::is_same<TP, TG>::value, "all-16-bit triples only");
+    return sizeof(TP) == 2 && sizeof(TG) == 2 && sizeof(TS) == 2 ? kVec16 : kVec;
+}
+
+// Run w of a call in the layout of its triple.
+template <typename TP, typename TG, typename TS, bool MIS>
+__device__ __forceinline__ void update_wave(const StepArgs& a, uint64_t w, uint32_t lane, bool has_coef, float coef)
+{
+    if constexpr (lane_elems<TP, TG, TS>() == kVec16) {
+        static_assert(std::is_same<TP, TS>::value && std::is_same<TP, TG>::value, "all-16-bit triples have one type");
+        update_run16<TP, MIS>(a, w, lane, has_coef, coef);
+    } else {
+        update_run<TP, TG, TS, MIS>(a, w, lane, has_coef, coef);
+    }
+}
+
+template <typename TP, typename TG, typename TS, bool MIS>
+__global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
+{
     const bool has_coef = a.coef != nullptr;
     const float coef = has_coef ? *a.coef : 1.0f;
     const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * LA_BLOCK + threadIdx.x;
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_BLOCK;
+
+    // Wave w owns run w: groups [64w, 64w + 64), 256 (all-16-bit triples 512)
+    // lane-contiguous elements per stream.  The grid is one-shot unless n exceeds LA_MAX_GRID runs.
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t nwaves = stride >> 6;
     for (uint64_t w = wave_uniform(tid >> 6); w * 64 < a.nvec; w += nwaves)
-        update_run16<TP, TG, MIS>(a, w, lane, has_coef, coef);
-    const uint64_t vec_end = a.head + a.nvec * kVec16;
+        update_wave<TP, TG, TS, MIS>(a, w, lane, has_coef, coef);
+
+    // Elements outside the aligned groups: [0, head) and [head + lane elements * nvec, n).
+    const uint64_t vec_end = a.head + a.nvec * lane_elems<TP, TG, TS>();
     const uint64_t nscalar = a.head + (a.n - vec_end);
     for (uint64_t s = tid; s < nscalar; s += stride) {
         const uint64_t e = s < a.head ? s : vec_end + (s - a.head);
@@ -406,7 +404,7 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw16_kernel(StepArgs a)
 // own reference adam_update call with its own scalars (the beta-power state
 // advances once per call) and its own scalar tail.  Waves [run_begin[s],
 // run_begin[s+1]) take the runs of segment s; then one wave per segment takes
-// its at most 21 elements outside the aligned groups.  Segments must not
+// its at most 29 elements outside the aligned groups.  Segments must not
 // overlap in memory.
 constexpr int kMaxSegs = 16;
 // Segments of any size go in a batch: with the wave index and the segment
@@ -438,13 +436,13 @@ __global__ __launch_bounds__(LA_BLOCK) void la_adamw_multi_kernel(MultiArgs a)
     if (w < runs) {
         uint32_t s = 0;
         while (w >= a.run_begin[s + 1]) ++s;
-        update_run<TP, TG, TS, MIS>(a.seg[s], w - a.run_begin[s], lane, has_coef, coef);
+        update_wave<TP, TG, TS, MIS>(a.seg[s], w - a.run_begin[s], lane, has_coef, coef);
         return;
     }
     const uint64_t s = w - runs;
     if (s >= a.count) return;
     const StepArgs& sa = a.seg[s];
-    const uint64_t vec_end = sa.head + sa.nvec * kVec;
+    const uint64_t vec_end = sa.head + sa.nvec * lane_elems<TP, TG, TS>();
     const uint64_t nscalar = sa.head + (sa.n - vec_end);
     if (lane < nscalar) {
         const uint64_t e = lane < sa.head ? lane : vec_end + (lane - sa.head);
@@ -637,7 +635,7 @@ bool dt_valid(int dt) { return dt == LA_F32 || dt == LA_BF16 || dt == LA_F16; }
 
 // First element index h in [0, vec) at which every pointer is aligned to a
 // full group of `vec` elements (4 elements: 16 bytes for fp32, 8 bytes for
-// 16-bit types), or -1 when the pointers disagree in phase.
+// 16-bit types; 8 elements of an all-16-bit triple: 16 bytes), or -1 when the pointers disagree in phase.
 int common_head(const uintptr_t* addr, const int* bytes, int count, int vec = kVec)
 {
     for (int h = 0; h < vec; ++h) {
@@ -654,7 +652,7 @@ int common_head(const uintptr_t* addr, const int* bytes, int count, int vec = kV
 // The head of a call whose streams disagree in phase, for the misphased form: the h in [0, vec) that
 // leaves the fewest bytes per element in misaligned accesses (p, m and v are
 // read and written, g is only read, the bf16 copy only written).
-int best_head(const uintptr_t* addr, const int* bytes, int count, int vec = kVec)
+int best_head(const uintptr_t* addr, const int* bytes, int count, int vec)
 {
     int best = 0, best_cost = INT32_MAX;
     for (int h = 0; h < vec; ++h) {
@@ -719,38 +717,18 @@ int launch(void (*kernel)(KArgs...), dim3 grid, dim3 block, uint32_t lds_bytes, 
 template <typename TP, typename TG, typename TS> constexpr uint32_t update_lds_bytes()
 {
     if (LA_UPDATE_LDS_OVERRIDE) return LA_UPDATE_LDS_BYTES;
-    if (std::is_same<TP, bf16_t>::value && std::is_same<TS, bf16_t>::value) return 8192;       // (bf16, bf16, bf16)
-    if (std::is_same<TP, f16_t>::value && std::is_same<TS, f16_t>::value) return 10240;       // (f16, f16, f16)
+    if (std::is_same<TP, bf16_t>::value && std::is_same<TS, bf16_t>::value) return 12288;      // (bf16, bf16, bf16)
     if (std::is_same<TP, float>::value && std::is_same<TG, float>::value) return 14336;       // (f32, f32, f32)
     return LA_UPDATE_LDS_BYTES;
-}
-
-// The all-16-bit path moves twice the bytes per wave, so it wants fewer
-// resident waves than the 4-element layout of the same triple.  Measured on
-// MI355X, C2 shape, 100 launches, three runs, ms per launch (4-element layout
-// at its own best cap / 8-element layout at 10, 11, 12, 13, 14 KiB reserved):
-// (bf16, bf16, bf16) 0.571-0.574 / 0.549-0.553, 0.547-0.551, 0.546-0.550,
-// 0.550-0.553, 0.560-0.561; (f16, f16, f16) 0.539-0.541 / 0.534-0.536,
-// 0.532-0.534, 0.531, 0.524-0.525, 0.524-0.526.  Kept: 12 KiB (13 waves per
-// CU) and 13 KiB (12).  LA_UPDATE16_LDS_BYTES, when defined, overrides both;
-// LA_WIDE16=0 restores the 4-element layout for these triples.
-#ifndef LA_WIDE16
-#define LA_WIDE16 1
-#endif
-template <typename T> constexpr uint32_t update16_lds_bytes()
-{
-#ifdef LA_UPDATE16_LDS_BYTES
-    return LA_UPDATE16_LDS_BYTES;
-#else
-    return std::is_same<T, bf16_t>::value ? 12288u : 13312u;
-#endif
 }
 
 // The multi kernel's waves first look up their segment and its arguments, a
 // latency that more resident waves hide better: at most 10 KiB (16 waves per
 // CU).  Measured on MI355X, a GPT-2 block's twelve tensors in one launch,
 // (f32, bf16, f32), step_with_grad_views: 30.4 us at 16 waves, 31.2 at 20,
-// 32.1 at 12, 31.3 uncapped.  LA_MULTI_LDS_BYTES, when defined, overrides it
+// 32.1 at 12, 31.3 uncapped; a Llama-3.1-8B layer's nine bf16 tensors with
+// bf16 moments, step: 457 us at 16 waves (8 elements per lane; 490 us with 4),
+// 466 at 20, 470 at 13, 485 at 12, 484 uncapped.  LA_MULTI_LDS_BYTES, when defined, overrides it
 // for every triple.
 template <typename TP, typename TG, typename TS> constexpr uint32_t multi_lds_bytes()
 {
@@ -761,54 +739,16 @@ template <typename TP, typename TG, typename TS> constexpr uint32_t multi_lds_by
 #endif
 }
 
-// Launch of la_adamw_kernel for the 4-element layout of `a`.
-template <typename TP, typename TG, typename TS> int launch4(const StepArgs& a, hipStream_t stream)
-{
-    const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * kVec));
-    // lanes needed: every wave takes one run of 64 groups
-    const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
-    const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
-    return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true> : la_adamw_kernel<TP, TG, TS, false>,
-                  dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
-                  update_lds_bytes<TP, TG, TS>(), stream, a);
-}
-
-// The all-16-bit path: the call's groups are re-laid out as 8-element groups.
-// Pointers that share a 4-element phase but not an 8-element one take the
-// misphased 8-element form too: 0.104 ms against 0.113 ms in the aligned
-// 4-element layout, (bf16, bf16, bf16) at 39 M elements.
-template <typename T> int launch16(const StepArgs& a4, hipStream_t stream)
-{
-    StepArgs a = a4;
-    const uintptr_t addr[5] = {reinterpret_cast<uintptr_t>(a.p), reinterpret_cast<uintptr_t>(a.g),
-                               reinterpret_cast<uintptr_t>(a.m), reinterpret_cast<uintptr_t>(a.v),
-                               reinterpret_cast<uintptr_t>(a.out)};
-    const int bytes[5] = {2, 2, 2, 2, 2};
-    int h = common_head(addr, bytes, a.out ? 5 : 4, kVec16);
-    a.misphased = h < 0;
-    if (h < 0) h = best_head(addr, bytes, a.out ? 5 : 4, kVec16);
-    if (static_cast<uint64_t>(h) >= a.tail_start) {
-        a.head = 0;
-        a.nvec = 0;
-    } else {
-        a.head = static_cast<uint64_t>(h);
-        a.nvec = (a.tail_start - a.head) / kVec16;
-    }
-    const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * kVec16));
-    const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
-    const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
-    return launch(a.misphased ? la_adamw16_kernel<T, T, T, true> : la_adamw16_kernel<T, T, T, false>,
-                  dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK),
-                  update16_lds_bytes<T>(), stream, a);
-}
-
 template <typename TP, typename TG, typename TS> struct StepLauncher {
     static int run(const StepArgs& a, hipStream_t stream)
     {
-        if constexpr (LA_WIDE16 && std::is_same<TP, TG>::value && std::is_same<TP, TS>::value &&
-                      !std::is_same<TP, float>::value)
-            return launch16<TP>(a, stream);
-        return launch4<TP, TG, TS>(a, stream);
+        const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * lane_elems<TP, TG, TS>()));
+        // lanes needed: every wave takes one run of 64 groups
+        const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
+        const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
+        return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true> : la_adamw_kernel<TP, TG, TS, false>,
+                      dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK), update_lds_bytes<TP, TG, TS>(),
+                      stream, a);
     }
 };
 
@@ -854,6 +794,11 @@ int prepare_step(int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, 
                                reinterpret_cast<uintptr_t>(p_bf16_out)};
     const int bytes[5] = {elem_bytes(p_dtype), elem_bytes(g_dtype), elem_bytes(s_dtype), elem_bytes(s_dtype), 2};
     const int count = p_bf16_out ? 5 : 4;
+    // elements per lane (lane_elems of the triple).  All-16-bit phases that agree
+    // modulo 4 elements but not 8 take the misphased 8-element form: 0.104 ms
+    // against 0.113 ms in an aligned 4-element layout, (bf16, bf16, bf16) at
+    // 39 M elements.
+    const int vec = bytes[0] == 2 && bytes[1] == 2 && bytes[2] == 2 ? kVec16 : kVec;
     for (int i = 0; i < count; ++i)
         if (addr[i] % static_cast<uintptr_t>(bytes[i]) != 0) return LA_EINVAL;
     if (clip_coef && (reinterpret_cast<uintptr_t>(clip_coef) & 3u)) return LA_EINVAL;
@@ -868,15 +813,15 @@ int prepare_step(int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, 
     a.coef = clip_coef;
     a.n = n;
     a.tail_start = n - n % 16;
-    int h = common_head(addr, bytes, count);
+    int h = common_head(addr, bytes, count, vec);
     a.misphased = h < 0;
-    if (h < 0) h = best_head(addr, bytes, count);
+    if (h < 0) h = best_head(addr, bytes, count, vec);
     if (static_cast<uint64_t>(h) >= a.tail_start) {
         a.head = 0;
         a.nvec = 0;
     } else {
         a.head = static_cast<uint64_t>(h);
-        a.nvec = (a.tail_start - a.head) / kVec;
+        a.nvec = (a.tail_start - a.head) / static_cast<uint64_t>(vec);
     }
     return LA_OK;
 }
