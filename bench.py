@@ -73,7 +73,8 @@ def read_traffic():
     return value, source
 
 
-UPDATE_KERNEL_RE = r"la_adamw_kernel<float, [^<>]*bf16_t, float>"
+# the one-shot launch on aligned streams: template arguments (p, g, state types, misphased, workgroup size)
+UPDATE_KERNEL_RE = r"la_adamw_kernel<float, [^<>]*bf16_t, float(?:, false(?:, 64)?)?>"
 READ_COUNTERS = ("TCC_EA0_RDREQ_128B_sum", "TCC_EA0_RDREQ_64B_sum", "TCC_EA0_RDREQ_32B_sum")
 WRITE_COUNTERS = ("TCC_EA0_WRREQ_sum", "TCC_EA0_WRREQ_64B_sum")
 
