@@ -224,9 +224,12 @@ int la_clip_coef(const double* sqnorm, float max_norm, float* coef, float* norm_
  * Replaces the runtime's chunk pipeline around the update: CPU fp32->bf16
  * cast + H2D (transformer_layer.py:297-305), grad D2H in chunks with
  * per-chunk events (:343-422) and the update thread consuming them (:453-493).
- * Here the host-resident arrays are copied in, updated on the GPU and copied
- * back, chunk by chunk, on three HIP streams (H2D, compute, D2H) so that
- * transfers in both directions overlap the update of other chunks.
+ * Here the update kernel reads and writes the host-resident arrays itself,
+ * over the host link, where they are page-locked coherent memory
+ * (hipHostMalloc's default) or go through such staging (below).  Other host
+ * arrays are copied in, updated on the GPU and copied back, chunk by chunk, on
+ * three HIP streams (H2D, compute, D2H) so that transfers in both directions
+ * overlap the update of other chunks.  The results are the same bit for bit.
  *
  * Placement: `on_host` has one bit per array.  A set bit means the array is
  * in host memory and streams through the device slots; a clear bit means it
@@ -269,7 +272,7 @@ int la_clip_coef(const double* sqnorm, float max_norm, float* coef, float* norm_
  *   or detach it with pinned = NULL.  While attached, la_pipeline_step copies
  *   every pageable host array through it: `threads` host threads copy each
  *   chunk into the page-locked twin of its slot and the results back out, and
- *   the copy engines only ever see page-locked memory.  Without it pageable
+ *   the device only ever sees page-locked memory.  Without it pageable
  *   arrays go through the HIP runtime's own bounce buffers.  Changing the
  *   attachment settles every queued call first.  No
  *   reference counterpart: the reference updates pageable state on the CPU.
@@ -287,10 +290,11 @@ typedef struct {
     float wall_ms;      /* first H2D start .. last D2H end; with staging, the whole call (host clock) */
     float h2d_ms;       /* span of the H2D stream (includes waits for free slots) */
     float compute_ms;   /* span of the compute stream */
-    float d2h_ms;       /* span of the D2H stream */
+    float d2h_ms;       /* span of the D2H stream (all three the launches' span where
+                           the kernel reads and writes host memory itself) */
     uint64_t h2d_bytes;
     uint64_t d2h_bytes;
-    uint32_t chunks;
+    uint32_t chunks;        /* ceil(n / chunk_elems) */
     float host_copy_ms;     /* time the host threads spent copying through the staging */
     uint64_t staged_bytes;  /* bytes they copied (both directions) */
 } la_pipeline_stats_t;

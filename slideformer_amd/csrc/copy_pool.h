@@ -63,6 +63,15 @@ struct Piece {
     uint64_t bytes;
 };
 
+// A list of at most this many bytes is copied by the calling thread alone: a
+// round with 15 workers takes ~45 us however little it copies.  Measured on
+// the MI355X host, one pageable step of 16,384 elements (192 KiB each way):
+// 84 us alone, 140-150 us with the workers; at 65,536 elements the same.
+#ifndef LA_COPY_ALONE_BYTES
+#define LA_COPY_ALONE_BYTES (512u << 10)
+#endif
+constexpr uint64_t kAloneBytes = LA_COPY_ALONE_BYTES;
+
 // run() hands a list of pieces to the workers and the calling thread and
 // returns when every piece is copied.  One run() at a time per pool.
 class CopyPool {
@@ -86,6 +95,14 @@ public:
     void run(const std::vector<Piece>& pieces)
     {
         if (pieces.empty()) return;
+        // few bytes: waking the workers takes longer than the copy
+        uint64_t bytes = 0;
+        for (const Piece& q : pieces) bytes += q.bytes;
+        if (bytes <= kAloneBytes) {
+            next_.store(0);
+            drain(pieces);
+            return;
+        }
         {
             std::lock_guard<std::mutex> g(mu_);
             job_ = &pieces;
@@ -122,7 +139,7 @@ private:
         }
 #if defined(__x86_64__)
         // nontemporal stores are weakly ordered: make them globally visible
-        // before run() reports the copy done (the copy engines read them next)
+        // before run() reports the copy done (the device reads them next)
         if (streamed) _mm_sfence();
 #endif
     }

@@ -38,6 +38,33 @@ inline bool device_accessible(const void* ptr)
 // Page-locked host memory, which the copy engines read and write directly.
 inline bool page_locked(const void* ptr) { return memory_type(ptr) == hipMemoryTypeHost; }
 
+// Whether kernels on `device` may read and write all of [ptr, ptr + bytes) in
+// host memory, at the same address: one page-locked allocation of that device,
+// mapped at its host address, and coherent (the kernels' accesses then bypass
+// the L2: nothing stale is read, and results are in host memory once the launch
+// is complete).  On this runtime plain, mapped and coherent allocations and
+// registrations are; any other flag (portable, write-combined, non-coherent)
+// can make the memory coarse-grained.
+inline bool kernel_reaches_host(const void* ptr, uint64_t bytes, int device)
+{
+    hipPointerAttribute_t a;
+    std::memset(&a, 0, sizeof(a));
+    unsigned flags = 0;
+    void* start = nullptr;
+    size_t size = 0;
+    const hipDeviceptr_t p = const_cast<void*>(ptr);
+    if (hipPointerGetAttributes(&a, ptr) != hipSuccess || a.type != hipMemoryTypeHost ||
+        hipHostGetFlags(&flags, p) != hipSuccess ||
+        hipPointerGetAttribute(&start, HIP_POINTER_ATTRIBUTE_RANGE_START_ADDR, p) != hipSuccess ||
+        hipPointerGetAttribute(&size, HIP_POINTER_ATTRIBUTE_RANGE_SIZE, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const uint64_t offset = static_cast<uint64_t>(static_cast<const char*>(ptr) - static_cast<const char*>(start));
+    return a.device == device && a.devicePointer == ptr && !(flags & ~(hipHostMallocMapped | hipHostMallocCoherent)) &&
+           offset <= size && bytes <= size - offset;
+}
+
 }  // namespace la_ptr
 
 #endif  // SLIDEFORMER_AMD_HIP_PTR_H

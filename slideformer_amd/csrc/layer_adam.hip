@@ -42,6 +42,7 @@
 
 #include "../../include/layer_adam.h"
 #include "hip_ptr.h"
+#include "link_step.h"
 #include "wave_io.h"
 
 // Update workgroup size.  One wave per workgroup: in a one-shot grid a
@@ -126,7 +127,27 @@
 #define LA_UPDATE_LDS_OVERRIDE 0
 #define LA_UPDATE_LDS_BYTES 13312
 #endif
-static_assert(LA_BLOCK % 64 == 0, "workgroups are whole waves");
+// Launch shape of the update on host memory (la_link::step): a few persistent
+// workgroups that grid-stride.  The host link is full with 128 waves in
+// flight (14 B of reads per element, 3.5 KB per wave and trip); more waves
+// only queue, and workgroups on more compute units take them from kernels that
+// run beside the update.  Measured on MI355X, GB/s read from / written to
+// page-locked memory at once, 64 Mi elements, all state on the host / moments
+// in HBM (workgroups x lanes):
+//   32 x 256: 55.9 / 47.9, 56.7 / 37.8   (kept)     128 x 64: 56.5 / 48.4, 54.8 / 36.5
+//   16 x 512: 52.0 / 44.5, 55.5 / 37.0              256 x 64: 56.5 / 48.4, 56.5 / 37.7
+//   32 x 512: 54.0 / 46.3, 52.9 / 35.3             1024 x 64: 49.4 / 42.4, 56.6 / 37.8
+//   64 x 64 : 51.2 / 43.9, 51.7 / 34.5     one-shot, 12 waves per CU: 49.5 / 42.4, 55.1 / 36.7
+// The copy engines move 48 GB/s each way at once, 57 one way alone.  An 8192^3
+// bf16 product beside it takes 1.5 ms (0.83 alone) with 32 x 256, 1.37 with
+// 16 x 512 and 2.3-2.5 with workgroups on all 256 compute units.
+#ifndef LA_LINK_BLOCK
+#define LA_LINK_BLOCK 256
+#endif
+#ifndef LA_LINK_GRID
+#define LA_LINK_GRID 32
+#endif
+static_assert(LA_BLOCK % 64 == 0 && LA_LINK_BLOCK % 64 == 0, "workgroups are whole waves");
 static_assert(static_cast<unsigned long long>(LA_MAX_GRID) * LA_BLOCK <= 0xffffffffull,
               "the grid size in work-items must fit the dispatch packet's 32 bits");
 
@@ -376,13 +397,13 @@ __device__ __forceinline__ void update_wave(const StepArgs& a, uint64_t w, uint3
     }
 }
 
-template <typename TP, typename TG, typename TS, bool MIS>
-__global__ __launch_bounds__(LA_BLOCK) void la_adamw_kernel(StepArgs a)
+template <typename TP, typename TG, typename TS, bool MIS, int BLOCK>
+__global__ __launch_bounds__(BLOCK) void la_adamw_kernel(StepArgs a)
 {
     const bool has_coef = a.coef != nullptr;
     const float coef = has_coef ? *a.coef : 1.0f;
-    const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * LA_BLOCK + threadIdx.x;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_BLOCK;
+    const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * BLOCK + threadIdx.x;
+    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * BLOCK;
 
     // Wave w owns run w: groups [64w, 64w + 64), 256 (all-16-bit triples 512)
     // lane-contiguous elements per stream.  The grid is one-shot unless n exceeds LA_MAX_GRID runs.
@@ -746,9 +767,22 @@ template <typename TP, typename TG, typename TS> struct StepLauncher {
         // lanes needed: every wave takes one run of 64 groups
         const uint64_t vec_lanes = (a.nvec + 63) / 64 * 64;
         const uint64_t work = vec_lanes > nscalar ? vec_lanes : nscalar;
-        return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true> : la_adamw_kernel<TP, TG, TS, false>,
+        return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true, LA_BLOCK>
+                                  : la_adamw_kernel<TP, TG, TS, false, LA_BLOCK>,
                       dim3(grid_for(work, LA_BLOCK, LA_MAX_GRID)), dim3(LA_BLOCK), update_lds_bytes<TP, TG, TS>(),
                       stream, a);
+    }
+};
+
+// The same kernel on host memory (see LA_LINK_GRID).
+template <typename TP, typename TG, typename TS> struct LinkLauncher {
+    static int run(const StepArgs& a, hipStream_t stream)
+    {
+        const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * lane_elems<TP, TG, TS>()));
+        const uint64_t work = a.nvec > nscalar ? a.nvec : nscalar;
+        return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true, LA_LINK_BLOCK>
+                                  : la_adamw_kernel<TP, TG, TS, false, LA_LINK_BLOCK>,
+                      dim3(grid_for(work, LA_LINK_BLOCK, LA_LINK_GRID)), dim3(LA_LINK_BLOCK), 0, stream, a);
     }
 };
 
@@ -784,9 +818,10 @@ int dispatch_triple(int p, int g, int s, Args&&... args)
 }
 
 // Check the pointers of one call and lay out its elements (everything of
-// StepArgs but the coefficients).  n > 0.
+// StepArgs but the coefficients).  n > 0.  `placement_known`: the caller has
+// looked the arrays' memory up, host memory among them.
 int prepare_step(int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, void* m, void* v, uint64_t n,
-                 uint16_t* p_bf16_out, const float* clip_coef, StepArgs& a)
+                 uint16_t* p_bf16_out, const float* clip_coef, StepArgs& a, bool placement_known = false)
 {
     if (!p || !g || !m || !v) return LA_EINVAL;
     const uintptr_t addr[5] = {reinterpret_cast<uintptr_t>(p), reinterpret_cast<uintptr_t>(g),
@@ -802,9 +837,9 @@ int prepare_step(int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, 
     for (int i = 0; i < count; ++i)
         if (addr[i] % static_cast<uintptr_t>(bytes[i]) != 0) return LA_EINVAL;
     if (clip_coef && (reinterpret_cast<uintptr_t>(clip_coef) & 3u)) return LA_EINVAL;
-    for (int i = 0; i < count; ++i)
+    for (int i = 0; i < count && !placement_known; ++i)
         if (!device_accessible(reinterpret_cast<const void*>(addr[i]))) return LA_EFAULT;
-    if (clip_coef && !device_accessible(clip_coef)) return LA_EFAULT;
+    if (clip_coef && !placement_known && !device_accessible(clip_coef)) return LA_EFAULT;
     a.p = p;
     a.g = g;
     a.m = m;
@@ -1059,6 +1094,20 @@ int scratch_on_current_device(int dev, double** out)
 }
 
 }  // namespace
+
+namespace la_link {
+
+int step(const la_scalars_t& sc, int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, void* m, void* v,
+         uint64_t n, uint16_t* p_bf16_out, const float* clip_coef, hipStream_t stream)
+{
+    StepArgs a;
+    const int rc = prepare_step(p_dtype, p, g_dtype, g, s_dtype, m, v, n, p_bf16_out, clip_coef, a, true);
+    if (rc != LA_OK) return rc;
+    set_coeffs(sc, a.k);
+    return dispatch_triple<LinkLauncher>(p_dtype, g_dtype, s_dtype, a, stream);
+}
+
+}  // namespace la_link
 
 // ---------------------------------------------------------------------------
 // C ABI

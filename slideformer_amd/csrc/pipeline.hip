@@ -2,7 +2,21 @@
 //
 // For optimizer state that lives in host RAM (the reference runtime's layout:
 // fp32 master and moments on the CPU, transformer_layer.py:192-196 and
-// layer_adam.py:161-173), one call streams the state through HBM in chunks:
+// layer_adam.py:161-173).  A call takes one of two paths.
+//
+// Direct path, whenever every host array of the call is page-locked and
+// reachable by kernels, or goes through the page-locked staging below: the
+// update kernel itself reads the host arrays over the link and writes the
+// results back, a few persistent workgroups at a time (la_link::step).  Reads
+// and writes share every moment of the launch, so there is nothing to fill or
+// drain, and the link runs at 56 GB/s in and 48 out at once where the copy
+// engines reach 48 each way.  Page-locked arrays take one launch per 64 Mi
+// elements.  Staged arrays go in sub-chunks of at most 1 Mi elements through a
+// ring of twins: host threads copy sub-chunk i in while they copy an earlier
+// one out and the kernel works on those between.
+//
+// Copy-engine path, for pageable arrays without staging and page-locked ones
+// that kernels cannot reach: the call streams the state through HBM in chunks:
 //
 //   h2d stream :  copy the host-resident arrays among p, m, v, g of chunk i into
 //                 slot i % S
@@ -20,13 +34,13 @@
 // the reference's scalar tail.  The caller owns the device staging memory.
 //
 // Pageable host arrays (the reference allocates its moments with plain
-// torch.zeros, layer_adam.py:161-173) cannot be reached by the copy engines
-// directly; the runtime would bounce them through small internal buffers at a
+// torch.zeros, layer_adam.py:161-173) cannot be reached by kernels or copy
+// engines directly; the runtime would bounce them through small internal buffers at a
 // fraction of the link rate.  With page-locked host staging attached
 // (la_pipeline_set_host_staging), each slot gets a page-locked twin: a pool of
-// host threads copies chunk i of every pageable array into the twin, the copy
-// engines move the twin, and after the copy-back the threads copy the results
-// out of the twin before chunk i + S reuses it.
+// host threads copies chunk i of every pageable array into the twin, the kernel
+// (or the copy engines) works on the twin, and afterwards the threads copy the
+// results out of the twin before a later chunk reuses it.
 //
 // Calls need not drain the pipeline.  The slot ring carries over from call to
 // call, so the runtime's one-call-per-chunk protocol (transformer_layer.py:
@@ -50,6 +64,7 @@
 #include "../../include/layer_adam.h"
 #include "copy_pool.h"
 #include "hip_ptr.h"
+#include "link_step.h"
 
 using la_host::CopyPool;
 using la_host::Piece;
@@ -65,20 +80,57 @@ using la_host::Piece;
 #define LA_PIPELINE_TRACE_MS 0.5
 #endif
 
+// Direct path: most elements per sub-chunk of staged arrays, fewest, twins in
+// the ring, and elements per launch on page-locked arrays.  A call is split in
+// 8 to overlap its host copies with the link, within those bounds: below 256 Ki
+// elements the rounds of the host threads (~45 us each) take longer than they
+// hide.  Measured on MI355X, pageable p, m, v and page-locked grads, us per
+// call at 65,536 / 262,144 / 1,048,576 / 4,194,304 elements: copy engines 262 /
+// 390 / 855 / 2680; direct, fewest 64 Ki 160 / 370 / 655 / 1470, 128 Ki 162 /
+// 240 / 640 / 1460, 256 Ki 162 / 236 / 497 / 1435 (kept), 512 Ki 160 / 235 /
+// 496 / 1500.  A Llama-3.1-8B layer in 32 Mi calls: copy engines 97.1 ms,
+// direct 64.4; within 3 % with sub-chunks of 0.5-4 Mi and 4-10 twins, bound by
+// the host's memory (the threads' and the device's traffic share it).
+// Page-locked arrays: a launch of 64 Mi runs ~17 ms, and other work on the
+// device gets a gap between launches.  Same layer, master page-locked, moments
+// in HBM: copy engines 26.8 ms, direct 23.3 (56 GB/s in).
+#ifndef LA_DIRECT_SUB
+#define LA_DIRECT_SUB (1ull << 20)
+#endif
+#ifndef LA_DIRECT_SUB_MIN
+#define LA_DIRECT_SUB_MIN (1ull << 18)
+#endif
+#ifndef LA_DIRECT_SLOTS
+#define LA_DIRECT_SLOTS 6
+#endif
+#ifndef LA_DIRECT
+#define LA_DIRECT 1  // 0: every call takes the copy-engine path
+#endif
+#ifndef LA_DIRECT_LAUNCH
+#define LA_DIRECT_LAUNCH (64ull << 20)
+#endif
+
+constexpr uint64_t kMaxSlots = 16;
+
 struct la_pipeline {
     int device = 0;
     uint64_t chunk = 0;
     int slots = 0;
     hipStream_t h2d = nullptr, comp = nullptr, d2h = nullptr;
     std::vector<hipEvent_t> ev_h2d, ev_comp, ev_d2h;
+    std::vector<hipEvent_t> ev_direct;  // direct path: the launch on each sub-slot
     hipEvent_t t_begin = nullptr, t_h2d_end = nullptr, t_comp_end = nullptr, t_end = nullptr, t_comp_begin = nullptr,
                t_d2h_begin = nullptr;
     // page-locked host staging for pageable arrays (caller-owned; null = none)
     char* host_staging = nullptr;
     uint64_t host_staging_bytes = 0;
+    bool host_staging_direct = false;  // kernels reach all of it
     std::unique_ptr<CopyPool> pool;
-    // the slot ring across calls: chunks issued so far; slot_used[s] once
-    // ev_d2h[s] has been recorded
+    // the slot ring across calls: whose slots it holds (the copy-engine path's,
+    // done at ev_d2h, or the direct path's, done at ev_direct) and how many;
+    // chunks issued so far; slot_used[s] once the slot's event has been recorded
+    bool ring_direct = false;
+    uint64_t ring_slots = 0;
     uint64_t issued = 0;
     std::vector<char> slot_used;
     // copy-outs owed per slot (staged arrays of a chunk whose call returned
@@ -86,10 +138,11 @@ struct la_pipeline {
     std::vector<std::vector<Piece>> owed;
     // host byte ranges [lo, hi) touched by calls since the last full sync
     std::vector<std::pair<uintptr_t, uintptr_t>> touched;
-    // device workspace and slot size of the last call: slot s of another
-    // layout can overlap slot s + 1 of this one
+    // memory and slot size of the ring: slot s of another layout can overlap
+    // slot s + 1 of this one
     const char* last_ws = nullptr;
     uint64_t last_slot_bytes = 0;
+    bool pending_direct = false;  // direct launches that no call has waited for yet
     uint64_t calls = 0;  // la_pipeline_step calls so far (the trace's call numbers)
 };
 
@@ -133,23 +186,28 @@ using la_ptr::page_locked;
 // Device (or managed / unified) memory, which the update may read and write in place.
 inline bool device_memory(const void* ptr) { return la_ptr::device_accessible(ptr); }
 
-// Host copies are split into pieces of at most this many bytes for the pool.
+// Host copies are split into pieces of at most this many bytes for the pool;
+// the direct path's smaller chunks into smaller pieces, so that every thread
+// gets some (12 MB in pieces of 256 KiB / 1 MiB on 16 threads: 143 / 117 GB/s).
 constexpr uint64_t kPieceBytes = 1ull << 20;
+constexpr uint64_t kDirectPieceBytes = 1ull << 18;
 
-void add_pieces(std::vector<Piece>& out, void* dst, const void* src, uint64_t bytes)
+void add_pieces(std::vector<Piece>& out, void* dst, const void* src, uint64_t bytes, uint64_t piece = kPieceBytes)
 {
     char* d = static_cast<char*>(dst);
     const char* s = static_cast<const char*>(src);
-    for (uint64_t o = 0; o < bytes; o += kPieceBytes)
-        out.push_back(Piece{d + o, s + o, std::min(kPieceBytes, bytes - o)});
+    for (uint64_t o = 0; o < bytes; o += piece) out.push_back(Piece{d + o, s + o, std::min(piece, bytes - o)});
 }
+
+// Complete once the results of the ring's slot s are in its twin.
+hipEvent_t slot_done(const la_pipeline* pl, uint64_t s) { return pl->ring_direct ? pl->ev_direct[s] : pl->ev_d2h[s]; }
 
 // Copy the results of slot s out of its page-locked twin once its copy-back
 // has landed (nothing to do when no copy-out is owed).
 int settle_slot(la_pipeline* pl, uint64_t s)
 {
     if (pl->owed[s].empty()) return LA_OK;
-    const hipError_t e = hipEventSynchronize(pl->ev_d2h[s]);
+    const hipError_t e = hipEventSynchronize(slot_done(pl, s));
     if (e != hipSuccess) return rc_of(e);
     pl->pool->run(pl->owed[s]);
     pl->owed[s].clear();
@@ -160,7 +218,7 @@ int settle_slot(la_pipeline* pl, uint64_t s)
 // order of issue, then the copy streams.
 int settle_all(la_pipeline* pl)
 {
-    const uint64_t S = static_cast<uint64_t>(pl->slots);
+    const uint64_t S = pl->ring_slots;
     for (uint64_t j = 0; j < S; ++j) {
         const int rc = settle_slot(pl, (pl->issued + j) % S);
         if (rc != LA_OK) return rc;
@@ -169,7 +227,26 @@ int settle_all(la_pipeline* pl)
     if (e == hipSuccess) e = hipStreamSynchronize(pl->comp);
     if (e == hipSuccess) e = hipStreamSynchronize(pl->d2h);
     pl->touched.clear();
+    pl->pending_direct = false;
     return rc_of(e);
+}
+
+// Make the ring the given one; another ring's slots, or another layout's,
+// share its memory and owe copy-outs, so that work is completed first.
+int enter_ring(la_pipeline* pl, bool direct, uint64_t slots, const char* base, uint64_t slot_bytes)
+{
+    if (pl->ring_slots == slots && pl->ring_direct == direct && pl->last_ws == base &&
+        pl->last_slot_bytes == slot_bytes)
+        return LA_OK;
+    const int rc = settle_all(pl);
+    if (rc != LA_OK) return rc;
+    pl->ring_direct = direct;
+    pl->ring_slots = slots;
+    pl->last_ws = base;
+    pl->last_slot_bytes = slot_bytes;
+    pl->issued = 0;
+    std::fill(pl->slot_used.begin(), pl->slot_used.end(), 0);
+    return LA_OK;
 }
 
 // After a failure part-way through a call, let the queued copies finish before
@@ -180,13 +257,14 @@ int drain_streams(la_pipeline* pl, int rc)
     (void)hipStreamSynchronize(pl->h2d);
     (void)hipStreamSynchronize(pl->comp);
     (void)hipStreamSynchronize(pl->d2h);
-    const uint64_t S = static_cast<uint64_t>(pl->slots);
+    const uint64_t S = pl->ring_slots;
     for (uint64_t j = 0; j < S; ++j) {
         std::vector<Piece>& o = pl->owed[(pl->issued + j) % S];
         if (!o.empty() && pl->pool) pl->pool->run(o);
         o.clear();
     }
     pl->touched.clear();
+    pl->pending_direct = false;
     return rc;
 }
 
@@ -197,9 +275,161 @@ bool overlaps(const std::vector<std::pair<uintptr_t, uintptr_t>>& a, uintptr_t l
     return false;
 }
 
+// One array of a call: where its element 0 is, bytes per element, whether it is
+// in host memory, whether it goes through the staging, read and written or one
+// of the two.
+struct Array {
+    char* base;
+    int bytes;
+    bool host, staged, in, out;
+};
+constexpr int kArrays = 5;  // p, m, v, g, the bf16 copy
+
+// Twins of the direct path: one region per staged array in each slot.
+uint64_t direct_layout(uint64_t sub, const Array* a, uint64_t* region)
+{
+    uint64_t off = 0;
+    for (int k = 0; k < kArrays; ++k) {
+        region[k] = off;
+        if (a[k].staged) off += round_up(sub * static_cast<uint64_t>(a[k].bytes), kAlign);
+    }
+    return off;
+}
+
+// The ring of a direct call.  A call without staged arrays uses no slots; it
+// leaves the ring of earlier direct calls as it is, since it only adds to the
+// one stream that they share.
+int enter_direct(la_pipeline* pl, const Array* a, bool staged)
+{
+    if (!staged) return pl->ring_direct || pl->ring_slots == 0 ? LA_OK : enter_ring(pl, true, 0, nullptr, 0);
+    uint64_t region[kArrays];
+    const uint64_t slot = direct_layout(std::min<uint64_t>(pl->chunk, LA_DIRECT_SUB), a, region);
+    // the staging holds at least `slots` slots of `chunk` elements of every host array
+    return enter_ring(pl, true, std::min<uint64_t>(LA_DIRECT_SLOTS, pl->host_staging_bytes / slot), pl->host_staging,
+                      slot);
+}
+
+int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtype, int s_dtype, const Array* a,
+                uint64_t n, const float* clip_coef, hipStream_t caller, bool synchronize, la_pipeline_stats_t* stats)
+{
+    const bool wait = synchronize || stats;
+    bool staged = false;
+    for (int k = 0; k < kArrays; ++k) staged |= a[k].staged;
+    uint64_t h2d_bytes = 0, d2h_bytes = 0, staged_bytes = 0;
+    for (int k = 0; k < kArrays; ++k) {
+        if (a[k].host && a[k].in) h2d_bytes += n * a[k].bytes;
+        if (a[k].host && a[k].out) d2h_bytes += n * a[k].bytes;
+    }
+    double host_copy_ms = 0.0;
+    std::vector<Piece> pieces;
+    auto host_copy = [&]() {
+        if (pieces.empty()) return;
+        const auto t = std::chrono::steady_clock::now();
+        pl->pool->run(pieces);
+        host_copy_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
+        for (const Piece& q : pieces) staged_bytes += q.bytes;
+        pieces.clear();
+    };
+    // slot s is free: its launch is complete, its owed copy-out among `pieces`
+    auto free_slot = [&](uint64_t s) -> hipError_t {
+        if (!pl->slot_used[s]) return hipSuccess;
+        const hipError_t e = hipEventSynchronize(pl->ev_direct[s]);
+        if (e != hipSuccess) return e;
+        pieces.insert(pieces.end(), pl->owed[s].begin(), pl->owed[s].end());
+        pl->owed[s].clear();
+        pl->slot_used[s] = 0;
+        return hipSuccess;
+    };
+#define LA_DIRECT_TRY(expr)                                       \
+    do {                                                          \
+        const hipError_t e_ = (expr);                             \
+        if (e_ != hipSuccess) return drain_streams(pl, rc_of(e_)); \
+    } while (0)
+
+    // What the caller queued before comes first: on the host where its threads
+    // read the arrays.  A call that waits, with nothing in flight, needs no
+    // stream of its own.
+    const bool own = !wait || staged || pl->pending_direct;
+    hipStream_t st = own ? pl->comp : caller;
+    LA_DIRECT_TRY(hipEventRecord(pl->t_begin, caller));
+    if (staged) LA_DIRECT_TRY(hipEventSynchronize(pl->t_begin));
+    else if (own) LA_DIRECT_TRY(hipStreamWaitEvent(st, pl->t_begin, 0));
+    if (stats && own) LA_DIRECT_TRY(hipEventRecord(pl->t_comp_begin, st));
+
+    uint64_t step = LA_DIRECT_LAUNCH;
+    uint64_t region[kArrays] = {};
+    const uint64_t S = pl->ring_slots;
+    if (staged) {
+        const uint64_t sub = std::min<uint64_t>(pl->chunk, LA_DIRECT_SUB);
+        (void)direct_layout(sub, a, region);
+        step = std::min(sub, std::max<uint64_t>(LA_DIRECT_SUB_MIN, round_up(n / 8, 16)));
+    }
+    for (uint64_t off = 0; off < n; off += step) {
+        const uint64_t k = std::min(step, n - off);
+        const uint64_t s = staged ? pl->issued % S : 0;
+        char* twin = nullptr;
+        if (staged) {
+            // slot s was freed by the previous sub-chunk; its own copy-in runs
+            // with the copy-out of the slot after it
+            if (pl->slot_used[s]) {
+                LA_DIRECT_TRY(free_slot(s));
+                host_copy();
+            }
+            twin = pl->host_staging + s * pl->last_slot_bytes;
+            if (S > 2) LA_DIRECT_TRY(free_slot((s + 1) % S));
+            for (int j = 0; j < kArrays; ++j)
+                if (a[j].staged && a[j].in)
+                    add_pieces(pieces, twin + region[j], a[j].base + off * a[j].bytes, k * a[j].bytes,
+                               kDirectPieceBytes);
+            host_copy();
+        }
+        char* at[kArrays];
+        for (int j = 0; j < kArrays; ++j)
+            at[j] = a[j].staged ? twin + region[j] : a[j].base ? a[j].base + off * a[j].bytes : nullptr;
+        const int rc = la_link::step(sc, p_dtype, at[0], g_dtype, at[3], s_dtype, at[1], at[2], k,
+                                     reinterpret_cast<uint16_t*>(at[4]), clip_coef, st);
+        if (rc != LA_OK) return drain_streams(pl, rc);
+        if (staged) {
+            LA_DIRECT_TRY(hipEventRecord(pl->ev_direct[s], st));
+            pl->slot_used[s] = 1;
+            pl->issued++;
+            for (int j = 0; j < kArrays; ++j)
+                if (a[j].staged && a[j].out)
+                    add_pieces(pl->owed[s], a[j].base + off * a[j].bytes, twin + region[j], k * a[j].bytes,
+                               kDirectPieceBytes);
+        }
+    }
+    LA_DIRECT_TRY(hipEventRecord(pl->t_end, st));
+    if (!wait) {
+        pl->pending_direct = true;
+        return LA_OK;
+    }
+    if (own) LA_DIRECT_TRY(hipStreamWaitEvent(caller, pl->t_end, 0));
+    // the copy-outs owed, earlier calls' included, in order of issue
+    for (uint64_t j = 0; j < S; ++j) {
+        LA_DIRECT_TRY(free_slot((pl->issued + j) % S));
+        host_copy();
+    }
+    LA_DIRECT_TRY(hipEventSynchronize(pl->t_end));
+#undef LA_DIRECT_TRY
+    pl->touched.clear();
+    pl->pending_direct = false;
+    if (stats) {
+        stats->h2d_bytes = h2d_bytes;
+        stats->d2h_bytes = d2h_bytes;
+        (void)hipEventElapsedTime(&stats->wall_ms, pl->t_begin, pl->t_end);
+        // one launch reads, updates and writes: the three spans are one
+        (void)hipEventElapsedTime(&stats->compute_ms, own ? pl->t_comp_begin : pl->t_begin, pl->t_end);
+        stats->h2d_ms = stats->d2h_ms = stats->compute_ms;
+        stats->staged_bytes = staged_bytes;
+        stats->host_copy_ms = static_cast<float>(host_copy_ms);
+    }
+    return LA_OK;
+}
+
 void destroy_events(la_pipeline* pl)
 {
-    for (auto* v : {&pl->ev_h2d, &pl->ev_comp, &pl->ev_d2h})
+    for (auto* v : {&pl->ev_h2d, &pl->ev_comp, &pl->ev_d2h, &pl->ev_direct})
         for (hipEvent_t e : *v)
             if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : {pl->t_begin, pl->t_h2d_end, pl->t_comp_end, pl->t_end, pl->t_comp_begin, pl->t_d2h_begin})
@@ -228,8 +458,8 @@ try {
     if (!pl) return LA_EINVAL;
     pl->chunk = chunk_elems;
     pl->slots = slots;
-    pl->slot_used.assign(static_cast<size_t>(slots), 0);
-    pl->owed.resize(static_cast<size_t>(slots));
+    pl->slot_used.assign(kMaxSlots, 0);
+    pl->owed.resize(kMaxSlots);
     hipError_t e = hipGetDevice(&pl->device);
     // default priority everywhere (hipStreamCreateWithFlags, no priority argument)
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&pl->h2d, hipStreamNonBlocking);
@@ -243,6 +473,11 @@ try {
         pl->ev_h2d.push_back(a);
         pl->ev_comp.push_back(b);
         pl->ev_d2h.push_back(c);
+    }
+    for (uint64_t i = 0; i < LA_DIRECT_SLOTS && e == hipSuccess; ++i) {
+        hipEvent_t a = nullptr;
+        e = hipEventCreateWithFlags(&a, hipEventDisableTiming);
+        pl->ev_direct.push_back(a);
     }
     for (hipEvent_t* t : {&pl->t_begin, &pl->t_h2d_end, &pl->t_comp_end, &pl->t_end, &pl->t_comp_begin, &pl->t_d2h_begin})
         if (e == hipSuccess) e = hipEventCreate(t);
@@ -291,6 +526,7 @@ int la_pipeline_set_host_staging(la_pipeline_t* pl, void* pinned, uint64_t bytes
     {
         const int rc = settle_all(pl);
         if (rc != LA_OK) return rc;
+        pl->ring_slots = 0;
     }
     if (!pinned) {
         pl->host_staging = nullptr;
@@ -310,6 +546,7 @@ int la_pipeline_set_host_staging(la_pipeline_t* pl, void* pinned, uint64_t bytes
     }
     pl->host_staging = base;
     pl->host_staging_bytes = bytes;
+    pl->host_staging_direct = la_ptr::kernel_reaches_host(base, bytes, pl->device);
     return LA_OK;
 }
 
@@ -385,7 +622,6 @@ try {
     hipStream_t caller = static_cast<hipStream_t>(after);
     uint64_t h2d_bytes = 0, d2h_bytes = 0, staged_bytes = 0;
     double host_copy_ms = 0.0;
-    std::vector<Piece> pieces;
 
     // Host bytes this call reads or writes.  If an earlier call that has not
     // been settled touched any of them (the same layer stepped again), settle
@@ -403,18 +639,43 @@ try {
     add_range(hg, gp, n * gb);
     add_range(ho, op, n * 2);
     bool clash = pl->touched.size() > 4096;
-    // another workspace or slot layout than the previous call's: the slots of
-    // the two layouts overlap, so earlier work must be finished first
-    if (pl->issued > 0 && (ws != pl->last_ws || L.slot_bytes != pl->last_slot_bytes)) clash = true;
     for (int r = 0; r < nranges && !clash; ++r) clash = overlaps(pl->touched, ranges[r].first, ranges[r].second);
     if (clash) {
         const int rc = settle_all(pl);
         if (rc != LA_OK) return rc;
     }
-    for (int r = 0; r < nranges; ++r) pl->touched.push_back(ranges[r]);
-    pl->last_ws = ws;
-    pl->last_slot_bytes = L.slot_bytes;
 
+    // The direct path: every host array through a twin, or within the kernels'
+    // reach and on whole elements (the copy engines take any address).
+    Array arrays[kArrays] = {{pp, pb, hp, st_p, true, true},
+                             {mp, sb, hm, st_m, true, true},
+                             {vp, sb, hv, st_v, true, true},
+                             {const_cast<char*>(gp), gb, hg, st_g, true, false},
+                             {op, 2, ho, st_o, false, true}};
+    bool direct = LA_DIRECT != 0 && (!staged || pl->host_staging_direct);
+    for (const Array& a : arrays)
+        if (a.host && !a.staged)
+            direct = direct && !misaligned(a.base, a.bytes) &&
+                     la_ptr::kernel_reaches_host(a.base, n * a.bytes, pl->device);
+    {
+        const int rc = direct ? enter_direct(pl, arrays, staged)
+                              : enter_ring(pl, false, S, ws, L.slot_bytes);
+        if (rc != LA_OK) return rc;
+    }
+    for (int r = 0; r < nranges; ++r) pl->touched.push_back(ranges[r]);
+    if (direct) {
+        const int rc = direct_step(pl, *sc, p_dtype, g_dtype, s_dtype, arrays, n, clip_coef, caller, synchronize != 0,
+                                   stats);
+        if (rc == LA_OK && stats) {
+            stats->chunks = static_cast<uint32_t>(nchunks);
+            if (staged)
+                stats->wall_ms = static_cast<float>(
+                    std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count());
+        }
+        return rc;
+    }
+
+    std::vector<Piece> pieces;
     auto host_copy = [&]() {
         const auto a = std::chrono::steady_clock::now();
         pl->pool->run(pieces);
@@ -567,6 +828,7 @@ try {
         if (e != hipSuccess) return rc_of(e);
         // t_end follows every earlier call's copy-backs on the same stream
         pl->touched.clear();
+        pl->pending_direct = false;
     }
     if (stats) {
         stats->h2d_bytes = h2d_bytes;

@@ -44,6 +44,14 @@ int main()
             if (check_round(pool, src, dst, piece, round)) return 1;
         }
     }
+    // lists too large for the calling thread alone (kAloneBytes)
+    {
+        CopyPool pool(6);
+        for (int round = 0; round < 20; ++round) {
+            std::vector<char> src(la_host::kAloneBytes + 1 + round * 30011), dst(src.size(), 0);
+            if (check_round(pool, src, dst, 5000 + round * 977, round)) return 1;
+        }
+    }
     // copies through the nontemporal path: every destination/source phase,
     // sizes just below and above its thresholds
     {

@@ -1,0 +1,164 @@
+"""The streaming pipeline's direct path (kernels on page-locked host memory)
+and the rule that chooses it, against the CPU checker, bit for bit."""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from slideformer_amd import LayerAdam, _lib
+from slideformer_amd.layer_adam import HostStreamer
+from tests import _hip as H
+
+pytestmark = pytest.mark.gpu
+
+HP = (1e-3, 0.9, 0.999, 1e-8, 0.01, True)
+# hipHostMalloc flags
+PORTABLE, MAPPED, WRITE_COMBINED, COHERENT, NONCOHERENT = 0x1, 0x2, 0x4, 0x40000000, 0x80000000
+
+
+class Case:
+    """One layer on the host: the same numbers for the library and the checker."""
+
+    def __init__(self, n, seed):
+        rng = np.random.default_rng(seed)
+        self.n = n
+        self.p = rng.normal(0, 0.02, n).astype(np.float32)
+        self.m = rng.normal(0, 1e-3, n).astype(np.float32)
+        self.v = np.abs(rng.normal(0, 1e-6, n)).astype(np.float32)
+        self.rng = rng
+        self.orc = O.OracleAdam(1e-3, (0.9, 0.999), 1e-8, 0.01, True)
+        self.ref = [self.p.copy(), self.m.copy(), self.v.copy()]
+
+    def grads(self):
+        return torch.from_numpy(self.rng.normal(0, 1e-3, self.n).astype(np.float32)).bfloat16()
+
+    def expect(self, step, g, lo=0, hi=None):
+        hi = self.n if hi is None else hi
+        p, m, v = (x[lo:hi] for x in self.ref)
+        self.orc.update(step, *HP, p, H.to_np_bits(g[lo:hi], "bf16"), m, v, g16="bf16")
+
+    def check(self, p, m, v, out=None):
+        for t, x in zip((p, m, v), self.ref):
+            assert np.array_equal(H.to_np_bits(t, "f32"), x.view(np.uint32))
+        if out is not None:
+            assert np.array_equal(H.to_np_bits(out, "bf16"), O.f32_to_bf16(self.ref[0]))
+
+
+def direct(stats):
+    """The direct path reports one span for the three stages; the copy-engine path one per stream."""
+    return stats.h2d_ms == stats.compute_ms == stats.d2h_ms
+
+
+def streamed(dev, **shape):
+    overlap = shape.pop("overlap", False)
+    adam = LayerAdam(lr=1e-3, weight_decay=0.01, overlap_host_chunks=overlap)
+    adam._streamers[dev] = HostStreamer(dev, **shape)
+    return adam
+
+
+def flagged(x, flags, shift=0):
+    """x in a hipHostMalloc allocation of the given flags, `shift` bytes off its start; the tensor and its owner."""
+    rt = _lib._hip()
+    ptr = ctypes.c_void_p()
+    assert rt.hipHostMalloc(ctypes.byref(ptr), x.nbytes + 64, flags) == 0
+    raw = np.frombuffer((ctypes.c_uint8 * (x.nbytes + 64)).from_address(ptr.value), dtype=np.uint8)
+    raw[shift:shift + x.nbytes] = x.view(np.uint8)
+    return raw, ptr
+
+
+@pytest.mark.parametrize("flags,shift,is_direct", [(0, 0, True), (MAPPED, 4, True), (COHERENT, 12, True),
+                                                   (PORTABLE, 0, False), (WRITE_COMBINED, 0, False),
+                                                   (NONCOHERENT, 0, False), (0, 2, False)])
+def test_route_of_page_locked_memory(flags, shift, is_direct, hip_device):
+    """Coherent page-locked state takes the direct path, at any element
+    alignment; coarse-grained memory and arrays that start inside an element
+    keep the copy engines, which take both.  Repeated steps with the host
+    rewriting the master in between: nothing stale is read."""
+    c = Case(70_001, flags % 97 + shift)
+    raw, ptr = flagged(c.p, flags, shift)
+    L = _lib.load()
+    handle = ctypes.c_void_p()
+    _lib.check(L.la_pipeline_create(16384, 3, ctypes.byref(handle)), "la_pipeline_create")
+    mask = _lib.LA_ON_HOST_P | _lib.LA_ON_HOST_G
+    ws = torch.empty(L.la_pipeline_workspace_bytes(16384, 3, 0, 1, 0, mask), dtype=torch.uint8, device=hip_device)
+    m, v = torch.from_numpy(c.m).to(hip_device), torch.from_numpy(c.v).to(hip_device)
+    opt = H.HipAdam(1e-3, (0.9, 0.999), 1e-8, 0.01, True)
+    for step in range(1, 6):
+        g = c.grads().pin_memory()
+        sc, st = _lib.LaScalars(), _lib.LaPipelineStats()
+        _lib.check(L.la_scalars(opt.id, step, *HP[:5], 1, ctypes.byref(sc)), "la_scalars")
+        print(f"route flags={flags:#x} shift={shift} step={step}", flush=True)
+        _lib.check(L.la_pipeline_step(handle, ctypes.byref(sc), 0, ptr.value + shift, 1, g.data_ptr(), 0, m.data_ptr(),
+                                      v.data_ptr(), c.n, None, mask, None, ws.data_ptr(), ws.numel(),
+                                      torch.cuda.current_stream().cuda_stream, 1, ctypes.byref(st)),
+                   "la_pipeline_step")
+        assert direct(st) == is_direct
+        c.expect(step, g)
+        now = raw[shift:shift + 4 * c.n].copy().view(np.uint32)
+        assert np.array_equal(now, c.ref[0].view(np.uint32)), step
+        c.ref[0] *= np.float32(-0.5)                       # the host's own write between steps
+        raw[shift:shift + 4 * c.n] = c.ref[0].view(np.uint8)
+    c.check(torch.from_numpy(c.ref[0]), m, v)
+    L.la_pipeline_destroy(handle)
+    del raw
+    _lib._hip().hipHostFree(ptr)
+
+
+# one sub-chunk, the smallest split, its remainder, and more sub-chunks than twins
+@pytest.mark.parametrize("n", [17, 65_536, 65_537, 8 * 65_536 + 5, 3_000_001, 9 * 1_048_576 + 3])
+@pytest.mark.parametrize("pageable", ["state", "grads"])
+def test_staged_sub_chunks(n, pageable, hip_device):
+    c = Case(n, n)
+    adam = streamed(hip_device, chunk_elems=4 * 1024 * 1024, slots=2, host_threads=5)
+    host = [torch.from_numpy(x.copy()) for x in (c.p, c.m, c.v)]
+    if pageable == "grads":
+        host = [t.pin_memory() for t in host]
+    out = torch.empty(n, dtype=torch.bfloat16, device=hip_device)
+    for step in (1, 2, 3):
+        g = c.grads()
+        adam.step_chunk(host[0], g if pageable == "grads" else g.pin_memory(), host[1], host[2],
+                        dict(adam.defaults, step=step), bf16_out=out)
+        assert direct(adam.last_stream_stats)
+        assert adam.last_stream_stats.staged_bytes == n * (2 if pageable == "grads" else 24)
+        c.expect(step, g)
+        c.check(*host, out)
+
+
+def test_queued_calls_of_every_route_on_one_pipeline(hip_device):
+    """Calls that return once queued, in turn page-locked (direct), pageable
+    through the twins (direct), pageable without staging and coarse-grained
+    (copy engines), on disjoint parts of one layer and then on the same parts
+    again: each switch completes what it must."""
+    n, part = 120_000, 20_000
+    c = Case(n, 5)
+    adam = streamed(hip_device, chunk_elems=4096, slots=3, overlap=True, host_threads=3)
+    streamer = adam._streamers[hip_device]
+    coarse, owner = flagged(c.p, PORTABLE)
+    kinds = ["locked", "staged", "locked", "unstaged", "staged", "coarse"]
+    parts = []
+    for i, kind in enumerate(kinds):
+        lo, hi = i * part, (i + 1) * part
+        p, m, v = (torch.from_numpy(x[lo:hi].copy()) for x in (c.p, c.m, c.v))
+        if kind in ("locked", "coarse"):
+            p, m, v = p.pin_memory(), m.pin_memory(), v.pin_memory()
+        if kind == "coarse":
+            p = torch.from_numpy(coarse[:4 * n].view(np.float32))[lo:hi]
+        parts.append((kind, lo, hi, p, m, v))
+    for step in (1, 2, 3):
+        g = c.grads()
+        gd = g.to(hip_device)
+        for repeat in range(2):                     # the second round meets unsettled bytes of the first
+            for kind, lo, hi, p, m, v in parts:
+                streamer.stage_pageable = kind not in ("unstaged", "coarse")
+                adam.step_chunk(p, gd[lo:hi], m, v, dict(adam.defaults, step=2 * step - 1 + repeat))
+                c.expect(2 * step - 1 + repeat, g, lo, hi)
+        adam.synchronize()
+        for kind, lo, hi, p, m, v in parts:
+            for t, x in zip((p, m, v), c.ref):
+                assert np.array_equal(H.to_np_bits(t, "f32"), x[lo:hi].view(np.uint32)), (step, kind)
+    del parts, p, m, v, t, adam, streamer, coarse
+    _lib._hip().hipHostFree(owner)
