@@ -25,7 +25,8 @@
 // them across the wave64 with DPP and across the 8 waves of a workgroup in
 // LDS, and writes one partial per workgroup to the caller's workspace; stage 2
 // (one workgroup) folds the partials in a fixed order and, optionally, writes
-// the clip coefficient.
+// the clip coefficient.  Up to LA_NORM_ONE elements stage 1 is one workgroup
+// and ends the call itself.
 
 #include <hip/hip_runtime.h>
 
@@ -69,6 +70,17 @@
 // About 8 waves per CU, each with 4 KB in flight per trip, read best.
 #ifndef LA_NORM_MAX_GRID
 #define LA_NORM_MAX_GRID 256
+#endif
+// Up to this many elements stage 1 is one workgroup, which ends the call
+// itself: folding one partial needs no second launch (~4 us of host issue, and
+// 2-4 us of GPU time that the one workgroup's extra trips use up at the limit).
+// Measured on MI355X, clip_grad_norm and step_chunk, us per step issued back to
+// back / waited for, one workgroup against two launches: 4096 elements 26.3 /
+// 40.0 against 29.4 / 42.8, 131,072 26.3 / 39.5 against 29.5 / 42.6, 262,144
+// 26.6 / 40.5 against 29.4 / 42.5, 524,288 26.7 / 43.0 against 29.3 / 42.0,
+// 1,048,576 40.6 / 62 against 29.0 / 42.8.
+#ifndef LA_NORM_ONE
+#define LA_NORM_ONE 131072
 #endif
 // Groups of 4 each lane of the grad-norm kernel loads per loop trip.
 #ifndef LA_NORM_UNROLL
@@ -539,6 +551,23 @@ struct NormArgs {
     float* norm_out;      // may be null
 };
 
+// The total of a norm call, in one thread.
+__device__ __forceinline__ void write_norm(const NormArgs& a, double total)
+{
+    const double sq = a.accumulate ? *a.sqnorm + total : total;
+    *a.sqnorm = sq;
+    if (a.coef) write_clip(sq, a.max_norm, a.coef, a.norm_out);
+}
+
+// End of stage 1: the workgroup's partial, or, on a grid of one workgroup, the
+// call's result.
+__device__ __forceinline__ void sqnorm_end(const NormArgs& a, double t)
+{
+    if (threadIdx.x != 0) return;
+    if (gridDim.x == 1) write_norm(a, t);
+    else a.partials[blockIdx.x] = t;
+}
+
 // One buffer's share of stage 1 for thread `tid` of `stride`: its aligned
 // groups of 4, walked from the top of the buffer down, then its scalar head
 // and remainder, added into `acc` in a fixed order.
@@ -587,8 +616,7 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormArgs a)
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_NORM_BLOCK;
     double acc = 0.0;
     sqnorm_buffer<TG, NT>(a.g, a.n, a.head, a.nvec, tid, stride, acc);
-    const double t = block_sum_f64(acc);
-    if (threadIdx.x == 0) a.partials[blockIdx.x] = t;
+    sqnorm_end(a, block_sum_f64(acc));
 }
 
 // Stage 1 over up to LA_NORM_MULTI_MAX buffers of one element type in one
@@ -599,7 +627,7 @@ struct NormMultiArgs {
     const void* g[LA_NORM_MULTI_MAX];
     uint64_t n[LA_NORM_MULTI_MAX], head[LA_NORM_MULTI_MAX], nvec[LA_NORM_MULTI_MAX];
     int32_t count;
-    double* partials;
+    NormArgs end;  // where the sum goes; its buffer fields are unused
 };
 
 template <typename TG, bool NT>
@@ -609,8 +637,7 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_multi_kernel(NormMult
     const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_NORM_BLOCK;
     double acc = 0.0;
     for (int b = 0; b < a.count; ++b) sqnorm_buffer<TG, NT>(a.g[b], a.n[b], a.head[b], a.nvec[b], tid, stride, acc);
-    const double t = block_sum_f64(acc);
-    if (threadIdx.x == 0) a.partials[blockIdx.x] = t;
+    sqnorm_end(a.end, block_sum_f64(acc));
 }
 
 // Stage 2, one workgroup: fold the stage-1 partials in a fixed order.  The
@@ -622,11 +649,7 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_finish(NormArgs a, ui
     double s = 0.0;
     for (uint32_t i = threadIdx.x; i < nparts; i += LA_NORM_BLOCK) s += a.partials[i];
     const double total = block_sum_f64(s);
-    if (threadIdx.x == 0) {
-        const double sq = a.accumulate ? *a.sqnorm + total : total;
-        *a.sqnorm = sq;
-        if (a.coef) write_clip(sq, a.max_norm, a.coef, a.norm_out);
-    }
+    if (threadIdx.x == 0) write_norm(a, total);
 }
 
 __global__ void la_clip_coef_kernel(const double* sqnorm, float max_norm, float* coef, float* norm_out)
@@ -701,6 +724,7 @@ uint32_t grid_for(uint64_t work, uint64_t block, uint64_t cap)
 
 uint32_t norm_grid(uint64_t n)
 {
+    if (n <= LA_NORM_ONE) return 1;
     const uint64_t groups = (n + kVec - 1) / kVec;
     return grid_for((groups + LA_NORM_UNROLL - 1) / LA_NORM_UNROLL, LA_NORM_BLOCK, LA_NORM_MAX_GRID);
 }
@@ -981,7 +1005,7 @@ int launch_norm(int g_dtype, const void* g, uint64_t n, void* workspace, uint64_
                     dim3(LA_NORM_BLOCK), 0, st, a);
         break;
     }
-    if (rc != LA_OK) return rc;
+    if (rc != LA_OK || grid == 1) return rc;
     return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, a, grid);
 }
 
@@ -1011,7 +1035,6 @@ int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void
 
     NormMultiArgs m;
     m.count = count;
-    m.partials = static_cast<double*>(workspace);
     for (int b = 0; b < LA_NORM_MULTI_MAX; ++b) {
         m.g[b] = nullptr;
         m.n[b] = m.head[b] = m.nvec[b] = 0;
@@ -1028,6 +1051,14 @@ int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void
         }
     }
     const uint32_t grid = norm_grid(total);
+    NormArgs a{};
+    a.partials = static_cast<double*>(workspace);
+    a.sqnorm = sqnorm;
+    a.accumulate = accumulate ? 1 : 0;
+    a.max_norm = max_norm;
+    a.coef = coef;
+    a.norm_out = norm_out;
+    m.end = a;
     // plain loads for the read that produces the coefficient, nontemporal otherwise
     const bool nt = !(coef && LA_NORM_CLIP_PLAIN);
     int rc;
@@ -1045,14 +1076,7 @@ int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void
                     dim3(LA_NORM_BLOCK), 0, st, m);
         break;
     }
-    if (rc != LA_OK) return rc;
-    NormArgs a{};
-    a.partials = m.partials;
-    a.sqnorm = sqnorm;
-    a.accumulate = accumulate ? 1 : 0;
-    a.max_norm = max_norm;
-    a.coef = coef;
-    a.norm_out = norm_out;
+    if (rc != LA_OK || grid == 1) return rc;
     return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, a, grid);
 }
 
