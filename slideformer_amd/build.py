@@ -76,7 +76,7 @@ def build_library(out: str = LIB_PATH, defines: dict | None = None, verbose: boo
 # many-trip loop then run at test sizes.  Same sources, same flags; only these
 # launch limits differ.
 SMALL_GRID_LIB = os.path.join(LIB_DIR, "libslideformer_amd_smallgrid.so")
-SMALL_GRID_DEFINES = {"LA_MAX_GRID": 64, "LA_NORM_MAX_GRID": 2, "LA_NORM_ONE": 16384}
+SMALL_GRID_DEFINES = {"LA_MAX_GRID": 64, "LA_NORM_MAX_GRID": 2, "LA_NORM_ONE": 16384, "LA_NORM_RUNS": 4096}
 
 
 # The update kernel's memory-ceiling probes (csrc/stream_probe.hip: its exact

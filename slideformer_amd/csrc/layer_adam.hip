@@ -107,9 +107,6 @@
 #ifndef LA_NORM_CLIP_PLAIN
 #define LA_NORM_CLIP_PLAIN 1
 #endif
-#ifndef LA_NORM_DESCENDING
-#define LA_NORM_DESCENDING 1
-#endif
 // Dynamic LDS reserved per update workgroup, unused by the kernel: it caps the
 // workgroups (= waves) resident per CU at 160 KiB / (reserved bytes), 12 for
 // 13 KiB.  Fewer streams in flight at once keep the HBM row buffers busier.
@@ -541,8 +538,6 @@ __device__ __forceinline__ void write_clip(double sq, float max_norm, float* coe
 }
 
 struct NormArgs {
-    const void* g;
-    uint64_t n, head, nvec;
     double* partials;     // one slot per stage-1 workgroup
     double* sqnorm;
     int32_t accumulate;
@@ -568,75 +563,110 @@ __device__ __forceinline__ void sqnorm_end(const NormArgs& a, double t)
     else a.partials[blockIdx.x] = t;
 }
 
-// One buffer's share of stage 1 for thread `tid` of `stride`: its aligned
-// groups of 4, walked from the top of the buffer down, then its scalar head
-// and remainder, added into `acc` in a fixed order.
-template <typename TG, bool NT>
-__device__ __forceinline__ void sqnorm_buffer(const void* g, uint64_t n, uint64_t head, uint64_t nvec, uint64_t tid,
-                                              uint64_t stride, double& acc)
+// Most runs of one launch: the last trip's run numbers, up to 8 waves x 256
+// workgroups x LA_NORM_UNROLL beyond it, stay below 2^32.  2^31 runs of 256
+// elements are 1 TiB of bf16 grads; the small-grid test build takes fewer.
+#ifndef LA_NORM_RUNS
+#define LA_NORM_RUNS (1ull << 31)
+#endif
+constexpr uint32_t kBeyond = 1u << 30;  // an offset outside every run's descriptor
+
+// Stage 1 over up to N buffers of one element type in one launch (N is 1 or
+// LA_NORM_MULTI_MAX).  The buffers' runs of 64 aligned groups are numbered one
+// after the other, each buffer from its top down, and wave w of W takes runs
+// w, w + W, ...: LA_NORM_UNROLL loads are in flight whatever buffers they fall
+// into, so small tensors and remainders cost no trip of their own.  The last
+// buffer comes first, so the front ones, which the update's first waves read,
+// are read last.  With one buffer both N give the same bits.  Bound by HBM
+// for large buffers, by the latency of a trip or two for small ones.  Measured
+// on MI355X, us per call (this launch and the fold's), bf16, against a walk in
+// which every thread took its share of each buffer in turn and its remainder
+// group by group: the 12 tensors of a GPT-2 block 7.5 against 11.8, 32 tensors
+// of 4099 elements 8.2 against 15.6, the 9 of a layer of hidden size 2048 (54 M)
+// 22.1 against 26.0, of 4096 (218 M, whole trips of the walk) 71.3 against 70.0;
+// one buffer of 7.1 M 6.5 against 7.0, of 218 M 69.4 against 68.9.
+template <int N> struct NormBuffers {
+    // buffer count - 1 - j of the call at index j
+    const void* g[N];
+    uint64_t n[N], head[N], nvec[N];
+    uint32_t run_end[N];  // runs of buffers 0 .. j
+    int32_t count;
+    NormArgs end;         // where the sum goes
+};
+
+template <typename TG, bool NT, int N>
+__global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N> a)
 {
-    // aligned group i of the walk -> group index in the buffer
-    auto group = [nvec](uint64_t i) { return LA_NORM_DESCENDING ? nvec - 1 - i : i; };
-    auto load = [g, head](uint64_t gidx, float (&x)[kVec]) { Io<TG>::template load4<NT>(g, head + gidx * kVec, x); };
-    uint64_t gi = tid;
-    for (; gi + (LA_NORM_UNROLL - 1) * stride < nvec; gi += LA_NORM_UNROLL * stride) {
-        float x[LA_NORM_UNROLL][kVec];
-#pragma unroll
-        for (int u = 0; u < LA_NORM_UNROLL; ++u) load(group(gi + u * stride), x[u]);
-#pragma unroll
-        for (int u = 0; u < LA_NORM_UNROLL; ++u)
-#pragma unroll
-            for (int j = 0; j < kVec; ++j) {
-                const double d = static_cast<double>(x[u][j]);
-                acc = __builtin_fma(d, d, acc);
-            }
-    }
-    for (; gi < nvec; gi += stride) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t w = static_cast<uint32_t>(
+        __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x * (LA_NORM_BLOCK / 64) + (threadIdx.x >> 6))));
+    const uint32_t waves = gridDim.x * (LA_NORM_BLOCK / 64);
+    const int count = N == 1 ? 1 : a.count;
+    const uint32_t runs = a.run_end[count - 1];
+    double acc = 0.0;
+    // the buffer of the run at hand: its runs [begin, end), its first aligned
+    // group, the groups of its last run, its end
+    int b = -1;
+    uint32_t begin = 0, end = 0, last = 0;
+    const TG *bottom = nullptr, *top = nullptr;
+    auto seek = [&](uint32_t r) {
+        while (r >= end && b + 1 < count) {
+            ++b;
+            begin = end;
+            end = a.run_end[b];
+            const uint64_t nvec = a.nvec[b];
+            bottom = static_cast<const TG*>(a.g[b]) + a.head[b];
+            top = bottom + nvec * kVec;
+            last = (static_cast<uint32_t>(nvec) - 1) % 64 + 1;
+        }
+    };
+    auto add = [&acc](const Raw4<TG>& raw) {
         float x[kVec];
-        load(group(gi), x);
+        raw.widen(x);
 #pragma unroll
         for (int j = 0; j < kVec; ++j) {
             const double d = static_cast<double>(x[j]);
             acc = __builtin_fma(d, d, acc);
         }
+    };
+    for (uint32_t r0 = w; r0 < runs;) {
+        seek(r0);
+        Raw4<TG> raw[LA_NORM_UNROLL];
+        // trips inside one buffer, before its last run, which may be partial
+        for (; r0 + (LA_NORM_UNROLL - 1) * waves + 1 < end; r0 += LA_NORM_UNROLL * waves) {
+            const TG* at = top - (static_cast<uint64_t>(r0 - begin) * 64 + lane + 1) * kVec;
+#pragma unroll
+            for (int u = 0; u < LA_NORM_UNROLL; ++u)
+                raw[u].template load_from<NT>(at - static_cast<uint64_t>(u) * waves * (64 * kVec));
+#pragma unroll
+            for (int u = 0; u < LA_NORM_UNROLL; ++u) add(raw[u]);
+        }
+        if (r0 >= runs) break;
+        // a trip that meets a buffer's end: every load through the descriptor of
+        // its own run, empty past the last run; lane l takes the l-th group from
+        // the run's top, or none (an offset beyond the descriptor)
+#pragma unroll
+        for (int u = 0; u < LA_NORM_UNROLL; ++u) {
+            const uint32_t r = r0 + u * waves;
+            seek(r);
+            const uint32_t groups = r + 1 < end ? 64u : r < end ? last : 0u;
+            const TG* lo = groups == 64 ? top - (static_cast<uint64_t>(r - begin) + 1) * (64 * kVec) : bottom;
+            raw[u].template load<NT ? kAux : 0>(
+                WaveIo<TG>::rsrc(lo, 0, groups * kVec),
+                lane < groups ? (groups - 1 - lane) * static_cast<uint32_t>(kVec * sizeof(TG)) : kBeyond);
+        }
+#pragma unroll
+        for (int u = 0; u < LA_NORM_UNROLL; ++u) add(raw[u]);
+        r0 += LA_NORM_UNROLL * waves;
     }
-    const uint64_t vec_end = head + nvec * kVec;
-    const uint64_t nscalar = head + (n - vec_end);
-    for (uint64_t s = tid; s < nscalar; s += stride) {
-        const uint64_t e = s < head ? s : vec_end + (s - head);
-        const double d = static_cast<double>(Io<TG>::load1(g, e));
-        acc = __builtin_fma(d, d, acc);
+    // at most 3 elements before and 3 after each buffer's groups, one wave per buffer
+    for (uint32_t j = w; j < static_cast<uint32_t>(count); j += waves) {
+        const uint64_t head = a.head[j], vec_end = head + a.nvec[j] * kVec;
+        if (lane < head + (a.n[j] - vec_end)) {
+            const double d = static_cast<double>(Io<TG>::load1(a.g[j], lane < head ? lane : vec_end + (lane - head)));
+            acc = __builtin_fma(d, d, acc);
+        }
     }
-}
-
-template <typename TG, bool NT>
-__global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormArgs a)
-{
-    const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * LA_NORM_BLOCK + threadIdx.x;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_NORM_BLOCK;
-    double acc = 0.0;
-    sqnorm_buffer<TG, NT>(a.g, a.n, a.head, a.nvec, tid, stride, acc);
-    sqnorm_end(a, block_sum_f64(acc));
-}
-
-// Stage 1 over up to LA_NORM_MULTI_MAX buffers of one element type in one
-// launch: every thread takes its share of each buffer in turn, so a buffer of
-// any size is spread over the whole grid, and the partials hold the sum over
-// all of them.
-struct NormMultiArgs {
-    const void* g[LA_NORM_MULTI_MAX];
-    uint64_t n[LA_NORM_MULTI_MAX], head[LA_NORM_MULTI_MAX], nvec[LA_NORM_MULTI_MAX];
-    int32_t count;
-    NormArgs end;  // where the sum goes; its buffer fields are unused
-};
-
-template <typename TG, bool NT>
-__global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_multi_kernel(NormMultiArgs a)
-{
-    const uint64_t tid = static_cast<uint64_t>(blockIdx.x) * LA_NORM_BLOCK + threadIdx.x;
-    const uint64_t stride = static_cast<uint64_t>(gridDim.x) * LA_NORM_BLOCK;
-    double acc = 0.0;
-    for (int b = 0; b < a.count; ++b) sqnorm_buffer<TG, NT>(a.g[b], a.n[b], a.head[b], a.nvec[b], tid, stride, acc);
     sqnorm_end(a.end, block_sum_f64(acc));
 }
 
@@ -954,6 +984,42 @@ void derive_scalars(HostState& s, uint64_t step, float lr, float b1, float b2, f
     out->step = s.step;
 }
 
+// Stage 1 over `count` <= N checked buffers on `grid` workgroups, and the fold
+// of its partials where they are more than one.
+template <int N>
+int launch_sqnorm(int g_dtype, const la_grad_buffer_t* bufs, int count, uint32_t grid, const NormArgs& end,
+                  hipStream_t st)
+{
+    NormBuffers<N> m{};
+    m.count = count;
+    m.end = end;
+    const int gb = elem_bytes(g_dtype);
+    uint32_t runs = 0;
+    for (int j = 0; j < count; ++j) {
+        const la_grad_buffer_t& q = bufs[count - 1 - j];
+        m.g[j] = q.g;
+        m.n[j] = q.n;
+        const uintptr_t addr = reinterpret_cast<uintptr_t>(q.g);
+        const int h = q.n > 0 ? common_head(&addr, &gb, 1) : -1;
+        if (h >= 0 && static_cast<uint64_t>(h) < q.n) {
+            m.head[j] = static_cast<uint64_t>(h);
+            m.nvec[j] = (q.n - m.head[j]) / kVec;
+        }
+        runs += static_cast<uint32_t>((m.nvec[j] + 63) / 64);
+        m.run_end[j] = runs;
+    }
+    // plain loads for the read that produces the coefficient, nontemporal otherwise
+    const bool nt = !(end.coef && LA_NORM_CLIP_PLAIN);
+    auto stage1 = [&](auto tag) {
+        using TG = decltype(tag);
+        return launch(nt ? la_sqnorm_kernel<TG, true, N> : la_sqnorm_kernel<TG, false, N>, dim3(grid),
+                      dim3(LA_NORM_BLOCK), 0, st, m);
+    };
+    const int rc = g_dtype == LA_F32 ? stage1(float{}) : g_dtype == LA_BF16 ? stage1(bf16_t{}) : stage1(f16_t{});
+    if (rc != LA_OK || grid == 1) return rc;
+    return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, end, grid);
+}
+
 int launch_norm(int g_dtype, const void* g, uint64_t n, void* workspace, uint64_t workspace_bytes,
                 double* sqnorm, int accumulate, float max_norm, float* coef, float* norm_out, hipStream_t st)
 {
@@ -970,43 +1036,18 @@ int launch_norm(int g_dtype, const void* g, uint64_t n, void* workspace, uint64_
         (coef && !device_accessible(coef)) || (norm_out && !device_accessible(norm_out)))
         return LA_EFAULT;
 
-    NormArgs a;
-    const uint32_t grid = norm_grid(n);
-    a.g = g;
-    a.n = n;
-    a.head = 0;
-    a.nvec = 0;
-    const uintptr_t addr = reinterpret_cast<uintptr_t>(g);
-    const int h = n > 0 ? common_head(&addr, &gb, 1) : -1;
-    if (h >= 0 && static_cast<uint64_t>(h) < n) {
-        a.head = static_cast<uint64_t>(h);
-        a.nvec = (n - a.head) / kVec;
+    if (n / 256 >= LA_NORM_RUNS) {
+        // more runs than the kernel's 32-bit run numbers hold: part by part
+        const uint64_t half = n / 2 / kVec * kVec;
+        const int rc = launch_norm(g_dtype, g, half, workspace, workspace_bytes, sqnorm, accumulate, max_norm, nullptr,
+                                   nullptr, st);
+        if (rc != LA_OK) return rc;
+        return launch_norm(g_dtype, static_cast<const char*>(g) + half * gb, n - half, workspace, workspace_bytes,
+                           sqnorm, 1, max_norm, coef, norm_out, st);
     }
-    a.partials = static_cast<double*>(workspace);
-    a.sqnorm = sqnorm;
-    a.accumulate = accumulate ? 1 : 0;
-    a.max_norm = max_norm;
-    a.coef = coef;
-    a.norm_out = norm_out;
-    // plain loads for the read that produces the coefficient, nontemporal otherwise
-    const bool nt = !(coef && LA_NORM_CLIP_PLAIN);
-    int rc;
-    switch (g_dtype) {
-    case LA_F32:
-        rc = launch(nt ? la_sqnorm_kernel<float, true> : la_sqnorm_kernel<float, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, a);
-        break;
-    case LA_BF16:
-        rc = launch(nt ? la_sqnorm_kernel<bf16_t, true> : la_sqnorm_kernel<bf16_t, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, a);
-        break;
-    default:
-        rc = launch(nt ? la_sqnorm_kernel<f16_t, true> : la_sqnorm_kernel<f16_t, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, a);
-        break;
-    }
-    if (rc != LA_OK || grid == 1) return rc;
-    return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, a, grid);
+    const la_grad_buffer_t buf{g, n};
+    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out};
+    return launch_sqnorm<1>(g_dtype, &buf, 1, norm_grid(n), end, st);
 }
 
 int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void* workspace,
@@ -1033,51 +1074,21 @@ int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void
     for (int b = 0; b < count; ++b)
         if (bufs[b].n > 0 && !device_accessible(bufs[b].g)) return LA_EFAULT;
 
-    NormMultiArgs m;
-    m.count = count;
-    for (int b = 0; b < LA_NORM_MULTI_MAX; ++b) {
-        m.g[b] = nullptr;
-        m.n[b] = m.head[b] = m.nvec[b] = 0;
-    }
-    for (int b = 0; b < count; ++b) {
-        const uint64_t n = bufs[b].n;
-        m.g[b] = bufs[b].g;
-        m.n[b] = n;
-        const uintptr_t addr = reinterpret_cast<uintptr_t>(bufs[b].g);
-        const int h = n > 0 ? common_head(&addr, &gb, 1) : -1;
-        if (h >= 0 && static_cast<uint64_t>(h) < n) {
-            m.head[b] = static_cast<uint64_t>(h);
-            m.nvec[b] = (n - m.head[b]) / kVec;
+    uint64_t runs = 0;
+    for (int b = 0; b < count; ++b) runs += bufs[b].n / 256 + 1;
+    if (runs > LA_NORM_RUNS) {
+        // more runs than the kernel's 32-bit run numbers hold: buffer by buffer
+        for (int b = 0; b < count; ++b) {
+            const bool final = b + 1 == count;
+            const int rc = launch_norm(g_dtype, bufs[b].g, bufs[b].n, workspace, workspace_bytes, sqnorm,
+                                       accumulate || b > 0, max_norm, final ? coef : nullptr,
+                                       final ? norm_out : nullptr, st);
+            if (rc != LA_OK) return rc;
         }
+        return LA_OK;
     }
-    const uint32_t grid = norm_grid(total);
-    NormArgs a{};
-    a.partials = static_cast<double*>(workspace);
-    a.sqnorm = sqnorm;
-    a.accumulate = accumulate ? 1 : 0;
-    a.max_norm = max_norm;
-    a.coef = coef;
-    a.norm_out = norm_out;
-    m.end = a;
-    // plain loads for the read that produces the coefficient, nontemporal otherwise
-    const bool nt = !(coef && LA_NORM_CLIP_PLAIN);
-    int rc;
-    switch (g_dtype) {
-    case LA_F32:
-        rc = launch(nt ? la_sqnorm_multi_kernel<float, true> : la_sqnorm_multi_kernel<float, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, m);
-        break;
-    case LA_BF16:
-        rc = launch(nt ? la_sqnorm_multi_kernel<bf16_t, true> : la_sqnorm_multi_kernel<bf16_t, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, m);
-        break;
-    default:
-        rc = launch(nt ? la_sqnorm_multi_kernel<f16_t, true> : la_sqnorm_multi_kernel<f16_t, false>, dim3(grid),
-                    dim3(LA_NORM_BLOCK), 0, st, m);
-        break;
-    }
-    if (rc != LA_OK || grid == 1) return rc;
-    return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, a, grid);
+    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out};
+    return launch_sqnorm<LA_NORM_MULTI_MAX>(g_dtype, bufs, count, norm_grid(total), end, st);
 }
 
 }  // namespace

@@ -243,6 +243,41 @@ template <typename Conv> struct WaveIo16 {
         __builtin_amdgcn_raw_buffer_store_b64(u32x2{lo, hi}, r, static_cast<int>(lane * 8), 0, kAuxSt);
     }
 };
+// 4 consecutive elements at a byte offset from a descriptor, as loaded, and
+// their widening apart from it: several loads can be in flight while scalar
+// code between them branches.  An offset beyond the descriptor reads zeros.
+template <typename T> struct Raw4;
+template <> struct Raw4<float> {
+    u32x4 u;
+    template <int AUX> __device__ __forceinline__ void load(rsrc_t r, uint32_t offset)
+    {
+        u = __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(offset), 0, AUX);
+    }
+    template <bool NT> __device__ __forceinline__ void load_from(const void* p) { u = vload<u32x4, NT>(p); }
+    __device__ __forceinline__ void widen(float (&x)[kVec]) const
+    {
+        x[0] = __uint_as_float(u.x); x[1] = __uint_as_float(u.y);
+        x[2] = __uint_as_float(u.z); x[3] = __uint_as_float(u.w);
+    }
+};
+template <typename Conv> struct Raw4x16 {
+    u32x2 u;
+    template <int AUX> __device__ __forceinline__ void load(rsrc_t r, uint32_t offset)
+    {
+        u = __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(offset), 0, AUX);
+    }
+    template <bool NT> __device__ __forceinline__ void load_from(const void* p) { u = vload<u32x2, NT>(p); }
+    __device__ __forceinline__ void widen(float (&x)[kVec]) const
+    {
+        x[0] = Conv::to_f32(u.x & 0xffffu);
+        x[1] = Conv::to_f32(u.x >> 16);
+        x[2] = Conv::to_f32(u.y & 0xffffu);
+        x[3] = Conv::to_f32(u.y >> 16);
+    }
+};
+template <> struct Raw4<bf16_t> : Raw4x16<ConvBf16> {};
+template <> struct Raw4<f16_t> : Raw4x16<ConvF16> {};
+
 template <> struct WaveIo<bf16_t> : WaveIo16<ConvBf16> {};
 template <> struct WaveIo<f16_t> : WaveIo16<ConvF16> {};
 

@@ -45,3 +45,70 @@ def test_norm_around_the_one_workgroup_limit(n, kind, hip_device):
         assert abs(got - want) <= 1e-12 * want
         coef, norm = O.clip_coef(got, 1.0)
         assert cn[0].item() == np.float32(coef) and cn[1].item() == np.float32(norm)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f32", "f16"])
+@pytest.mark.parametrize("sizes", [(5, 0, 3), (256, 1, 255, 257), (0, 0, 0), (4099,) * 32, (700_001, 3, 1_048_576, 9),
+                                   (1_500_000, 64, 131_073, 2_000_003)])
+def test_norm_over_buffers_whose_runs_share_trips(sizes, kind, hip_device):
+    """la_grad_norm_multi numbers the 256-element runs of all buffers in one
+    sequence: empty buffers, buffers of scalars only, partial runs and odd
+    starts, on one workgroup and on many; also a sum within 1e-12 when the
+    buffers are given in the other order, and single buffers with the bits of
+    la_grad_norm_clip."""
+    L = _lib.load()
+    bufs = [(torch.randn(n + 8, device=hip_device) * 1e-2).to(H.TD[kind])[k % 4:k % 4 + n]
+            for k, n in enumerate(sizes)]
+    exact = sum(O.grad_sqnorm(_bits(g, kind), None if kind == "f32" else kind) for g in bufs if g.numel())
+    need = L.la_grad_sqnorm_workspace(max(1, sum(sizes)))
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def run(order):
+        ws = torch.full((need // 8,), float("nan"), dtype=torch.float64, device=hip_device)
+        sq = torch.full((1,), float("nan"), dtype=torch.float64, device=hip_device)
+        cn = torch.zeros(2, device=hip_device)
+        flat = [x for g in order for x in (g.data_ptr(), g.numel())]
+        arr = ctypes.cast((ctypes.c_uint64 * len(flat))(*flat), ctypes.POINTER(_lib.LaGradBuffer))
+        _lib.check(L.la_grad_norm_multi(H.CODE[kind], arr, len(order), ws.data_ptr(), need, sq.data_ptr(), 0, 0.5,
+                                        cn.data_ptr(), cn.data_ptr() + 4, stream), "la_grad_norm_multi")
+        return sq.item(), cn
+
+    print(f"multi norm {sizes[:6]} {kind}", flush=True)
+    for order in (bufs, bufs[::-1]):
+        got, cn = run(order)
+        assert abs(got - exact) <= 1e-12 * exact
+        coef, norm = O.clip_coef(got, 0.5)
+        assert cn[0].item() == np.float32(coef) and cn[1].item() == np.float32(norm)
+    for g in bufs:
+        if g.numel():
+            assert run([g])[0] == H.norm_clip(g, 0.5)[0].item()
+
+
+def test_norms_of_more_runs_than_one_launch_numbers(hip_device):
+    """The small-grid build numbers at most 4096 runs per launch (the product
+    build 2^31): a larger buffer is summed in parts and a larger list buffer by
+    buffer, to the same 1e-12, with the coefficient written once."""
+    L = H.load_small_grid()
+    stream = torch.cuda.current_stream().cuda_stream
+    ws = torch.full((2,), float("nan"), dtype=torch.float64, device=hip_device)
+    big = (torch.randn(5_000_009, device=hip_device) * 1e-2).bfloat16()[1:]
+    bufs = [big, big[:700_001], big[3:2_000_000], big[:0], big[5:10]]
+    for which in ("single", "multi"):
+        sq = torch.full((1,), float("nan"), dtype=torch.float64, device=hip_device)
+        cn = torch.zeros(2, device=hip_device)
+        if which == "single":
+            exact = O.grad_sqnorm(_bits(big, "bf16"), "bf16")
+            rc = L.la_grad_norm_clip(1, big.data_ptr(), big.numel(), ws.data_ptr(), 16, sq.data_ptr(), 0, 0.5,
+                                     cn.data_ptr(), cn.data_ptr() + 4, stream)
+        else:
+            exact = sum(O.grad_sqnorm(_bits(g, "bf16"), "bf16") for g in bufs if g.numel())
+            flat = [x for g in bufs for x in (g.data_ptr(), g.numel())]
+            arr = ctypes.cast((ctypes.c_uint64 * len(flat))(*flat), ctypes.POINTER(_lib.LaGradBuffer))
+            rc = L.la_grad_norm_multi(1, arr, len(bufs), ws.data_ptr(), 16, sq.data_ptr(), 0, 0.5, cn.data_ptr(),
+                                      cn.data_ptr() + 4, stream)
+        assert rc == 0
+        got = sq.item()
+        print(f"norm in parts, {which}", flush=True)
+        assert abs(got - exact) <= 1e-12 * exact
+        coef, norm = O.clip_coef(got, 0.5)
+        assert cn[0].item() == np.float32(coef) and cn[1].item() == np.float32(norm)
