@@ -9,6 +9,7 @@ There is no fallback: if the library is missing, ``load()`` raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 import weakref
@@ -18,6 +19,9 @@ import torch  # noqa: F401  (binds the HIP runtime before the library is loaded)
 
 # where slideformer_amd/build.py writes the library
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libslideformer_amd.so")
+
+# where it writes the native host module
+HOST_CALLS_PATH = os.path.join(os.path.dirname(LIB_PATH), "_host_calls.so")
 
 # LA_ABI_VERSION of include/layer_adam.h that these bindings declare
 ABI_VERSION = 9
@@ -217,6 +221,29 @@ def load(path: str | None = None):
                 "with `python -m slideformer_amd.build`")
         _lib = _declare(raw)
         return _lib
+
+
+_host_calls = None
+
+
+def host_calls():
+    """The native host module (csrc/host_calls.cpp), bound once to the loaded
+    library.  Raises ImportError if it has not been built."""
+    global _host_calls
+    if _host_calls is None:
+        L = load()
+        with _lock:
+            if _host_calls is None:
+                if not os.path.exists(HOST_CALLS_PATH):
+                    raise ImportError(f"{HOST_CALLS_PATH} not found; build it with `python -m slideformer_amd.build`")
+                spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS_PATH)
+                module = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(module)
+                module.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
+                    L.la_adam_update, L.la_adam_update_multi, L.la_grad_sqnorm, L.la_grad_norm_clip,
+                    L.la_grad_norm_multi)))
+                _host_calls = module
+    return _host_calls
 
 
 def check(rc: int, what: str) -> None:

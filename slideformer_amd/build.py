@@ -115,9 +115,45 @@ def build_c_driver(verbose: bool = False) -> str:
     return C_DRIVER
 
 
+# The CPython module of the host side of calls on HIP tensors (plain C++ against
+# torch's headers; it reaches the library through addresses bound at run time).
+HOST_CALLS_SRC = os.path.join(CSRC, "host_calls.cpp")
+HOST_CALLS = os.path.join(LIB_DIR, "_host_calls.so")
+
+
+def build_host_calls(verbose: bool = False) -> str:
+    """Compile csrc/host_calls.cpp with g++ against torch's and Python's headers."""
+    import sysconfig
+
+    import torch
+
+    gxx = shutil.which("g++")
+    if gxx is None:
+        raise RuntimeError("g++ not found")
+    os.makedirs(LIB_DIR, exist_ok=True)
+    root = os.path.dirname(torch.__file__)
+    cmd = [gxx, "-std=c++17", "-O2", "-Wall", "-fPIC", "-shared", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-isystem", os.path.join(root, "include"),
+           "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           "-isystem", sysconfig.get_paths()["include"], HOST_CALLS_SRC,
+           "-L", os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10",
+           f"-Wl,-rpath,{os.path.join(root, 'lib')}", "-o", HOST_CALLS + ".tmp"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        sys.stderr.write(res.stdout + res.stderr)
+        raise RuntimeError(f"g++ failed with code {res.returncode}")
+    os.replace(HOST_CALLS + ".tmp", HOST_CALLS)
+    return HOST_CALLS
+
+
 def build_all(verbose: bool = False) -> list:
-    """The product library, the small-grid test build, the stream probes and the C test driver."""
+    """The product library, the native host module, the small-grid test build, the stream probes and the C test
+    driver."""
     return [build_library(verbose=verbose),
+            build_host_calls(verbose=verbose),
             build_library(out=SMALL_GRID_LIB, defines=SMALL_GRID_DEFINES, verbose=verbose),
             build_library(out=PROBE_LIB, sources=PROBE_SOURCES, verbose=verbose),
             build_c_driver(verbose=verbose)]

@@ -224,41 +224,6 @@ def _unsupported(p, g, s) -> RuntimeError:
         f"and state type {_DTYPE_NAME.get(s, s)} is not supported on current hardware")
 
 
-def _segments(entries):
-    """The la_segment_t array of one la_adam_update_multi call over the
-    (params, grads, exp_avg, exp_avg_sq) entries, or None when they cannot go
-    in one: one HIP device, one registered dtype triple, contiguous, matching
-    sizes, and no two tensors written by the update overlapping.  One pass;
-    the array is built as six uint64 per segment (the layout of la_segment_t:
-    p, g, m, v, p_bf16_out, n)."""
-    p0, g0, m0, _ = entries[0]
-    if not p0.is_cuda:
-        return None
-    pdt, gdt, sdt = p0.dtype, g0.dtype, m0.dtype
-    if (pdt, gdt, sdt) not in SUPPORTED_TRIPLES:
-        return None
-    dev = p0.get_device()
-    pe, se = p0.element_size(), m0.element_size()
-    flat, spans = [], []
-    for p, g, m, v in entries:
-        n = p.numel()
-        if (g.numel() != n or m.numel() != n or v.numel() != n
-                or p.dtype != pdt or g.dtype != gdt or m.dtype != sdt or v.dtype != sdt
-                or not (p.is_contiguous() and g.is_contiguous() and m.is_contiguous() and v.is_contiguous())
-                or p.get_device() != dev or g.get_device() != dev or m.get_device() != dev
-                or v.get_device() != dev):
-            return None
-        pp, mp, vp = p.data_ptr(), m.data_ptr(), v.data_ptr()
-        flat += (pp, g.data_ptr(), mp, vp, 0, n)
-        if n:
-            spans += ((pp, pp + n * pe), (mp, mp + n * se), (vp, vp + n * se))
-    spans.sort()
-    for a, b in zip(spans, spans[1:]):
-        if a[1] > b[0]:
-            return None
-    return ctypes.cast((ctypes.c_uint64 * len(flat))(*flat), ctypes.POINTER(_lib.LaSegment))
-
-
 def _torch_stream(stream, device):
     """The stream a call runs on, as a torch stream object (None = current stream;
     a raw hipStream_t handle is wrapped), so that scratch tensors can be
@@ -281,50 +246,15 @@ def _norm_workspace_elems(lib) -> int:
     return _norm_elems
 
 
-def _norm_runs(lib, grads, work, nwork, sqnorm, accumulate, max_norm, cn, handle):
-    """The sum of squares of ``grads`` into the float64 at ``sqnorm`` (added to
-    it when ``accumulate``): runs of one dtype, at most LA_NORM_MULTI_MAX
-    buffers each, one library call (two launches) per run, later runs adding
-    to the earlier ones: la_grad_norm_multi for a run of several buffers,
-    la_grad_sqnorm / la_grad_norm_clip for a run of one.  With ``cn`` (address
-    of two fp32: coef, norm) the last call also writes the clip coefficient."""
-    runs = []
-    for g in grads:
-        if runs and runs[-1][0].dtype == g.dtype and len(runs[-1]) < _lib.LA_NORM_MULTI_MAX:
-            runs[-1].append(g)
-        else:
-            runs.append([g])
-    for i, run in enumerate(runs):
-        last = cn is not None and i == len(runs) - 1
-        acc = int(accumulate or i > 0)
-        code = _DTYPE_CODE[run[0].dtype]
-        if len(run) == 1:
-            # one buffer: the single-buffer entry points (the same bits, a smaller launch)
-            g = run[0]
-            if last:
-                rc = lib.la_grad_norm_clip(code, g.data_ptr(), g.numel(), work, nwork * 8, sqnorm, acc, max_norm, cn,
-                                           cn + 4, handle)
-            else:
-                rc = lib.la_grad_sqnorm(code, g.data_ptr(), g.numel(), work, nwork * 8, sqnorm, acc, handle)
-            _lib.check(rc, "la_grad_sqnorm")
-            continue
-        flat = []
-        for g in run:
-            flat += (g.data_ptr(), g.numel())
-        bufs = ctypes.cast((ctypes.c_uint64 * len(flat))(*flat), ctypes.POINTER(_lib.LaGradBuffer))
-        rc = lib.la_grad_norm_multi(code, bufs, len(run), work, nwork * 8, sqnorm, acc, max_norm,
-                                    cn if last else None, cn + 4 if last else None, handle)
-        _lib.check(rc, "la_grad_norm_multi")
-
-
 def _check_grads(grads, device):
-    for g in grads:
-        if g.device != device:
+    """Raise for the first grad that the norm does not take; ``device`` is a HIP device."""
+    index = device.index if device.index is not None else -1     # a tensor's device has an index
+    bad = _lib.host_calls().check_grads(grads, index)
+    if bad is not None:
+        g, why = grads[bad[0]], bad[1]
+        if why == 0:
             raise RuntimeError(f"grad on {g.device}, expected {device}: all grads must be on one device")
-        if not g.is_contiguous():
-            raise RuntimeError("grads must be contiguous")
-        if g.dtype not in _DTYPE_CODE:
-            raise RuntimeError(f"unsupported grad dtype {g.dtype}")
+        raise RuntimeError("grads must be contiguous" if why == 1 else f"unsupported grad dtype {g.dtype}")
 
 
 class LayerAdam:
@@ -410,6 +340,7 @@ class LayerAdam:
         # loads the HIP library and fails loudly if it is missing.  cpu_adam is
         # the module with the reference extension's three functions.
         self.lib = _lib.load()
+        self._host = _lib.host_calls()
         self.cpu_adam = cpu_adam_compat
         # The reference always uses id 0 (layer_adam.py:62), so a second
         # instance would reset the first one's beta-power state; each instance
@@ -599,6 +530,23 @@ class LayerAdam:
                     params, grads, exp_avg, exp_avg_sq, *, bf16_out=None, clip_coef=None,
                     stream=None):
         """One reference ``adam_update`` call (cpu_adam_impl.cpp:220-270) on the MI355X."""
+        index = params.get_device()
+        if index >= 0 and index == torch.cuda.current_device():
+            # tensors that pass every check below, on the current device, go straight to the library
+            rc = self._host.update(self.optimizer_id, int(step), lr, beta1, beta2, eps, weight_decay, bias_correction,
+                                   index, _stream_handle(stream, params.device), params, grads, exp_avg, exp_avg_sq,
+                                   bf16_out, clip_coef)
+            if rc is not None:
+                if rc:
+                    _lib.check(rc, "la_adam_update")
+                return
+        self._checked_update(step, lr, beta1, beta2, eps, weight_decay, bias_correction, params, grads, exp_avg,
+                             exp_avg_sq, bf16_out, clip_coef, stream, not self.overlap_host_chunks)
+
+    def _checked_update(self, step, lr, beta1, beta2, eps, weight_decay, bias_correction, params, grads, exp_avg,
+                        exp_avg_sq, bf16_out, clip_coef, stream, synchronize):
+        """``adam_update`` with every check in the reference's order.  ``synchronize``: host tensors' results are
+        complete on return (otherwise the caller synchronizes the streamers)."""
         # contiguity checks of cpu_adam_impl.cpp:234-237
         if not params.is_contiguous():
             raise RuntimeError("params must be contiguous")
@@ -640,7 +588,7 @@ class LayerAdam:
             raise RuntimeError(f"params/grads/states must be on one device, got {sorted(map(str, gpu_devs))}")
         self._host_update(step, lr, beta1, beta2, eps, weight_decay, bias_correction, params,
                           grads, exp_avg, exp_avg_sq, bf16_out, clip_coef, stream, n,
-                          gpu_devs.pop() if gpu_devs else None)
+                          gpu_devs.pop() if gpu_devs else None, synchronize)
 
     def _codes(self, params, grads, exp_avg):
         key = (params.dtype, grads.dtype, exp_avg.dtype)
@@ -672,10 +620,10 @@ class LayerAdam:
         _lib.check(rc, "la_adam_update")
 
     def _host_update(self, step, lr, beta1, beta2, eps, weight_decay, bias_correction, params,
-                     grads, exp_avg, exp_avg_sq, bf16_out, clip_coef, stream, n, gpu):
-        """Some arrays in host memory: stream those through HBM with the native
-        chunk pipeline (la_pipeline_step), the others are used in place on
-        ``gpu``; returns after completion, as the reference's CPU call does."""
+                     grads, exp_avg, exp_avg_sq, bf16_out, clip_coef, stream, n, gpu, synchronize):
+        """Some arrays in host memory: the native pipeline (la_pipeline_step)
+        streams those, the others are used in place on ``gpu``; with
+        ``synchronize`` returns after completion, as the reference's CPU call does."""
         if not torch.cuda.is_available():
             raise RuntimeError("LayerAdam needs a HIP device (MI355X); there is no CPU arithmetic path")
         sc = self._scalars(step, lr, beta1, beta2, eps, weight_decay, bias_correction)
@@ -691,12 +639,11 @@ class LayerAdam:
             on_host = _placement(params, grads, exp_avg, exp_avg_sq, bf16_out)
             self.last_stream_stats = streamer.step(
                 sc, pc, params, gc, grads, sc_, exp_avg, exp_avg_sq, n, bf16_out, on_host,
-                clip_coef, _stream_handle(stream, device), synchronize=not self.overlap_host_chunks)
+                clip_coef, _stream_handle(stream, device), synchronize=synchronize)
 
     # ------------------------------------------------------------------
     # steps (layer_adam.py:270-468)
     # ------------------------------------------------------------------
-    @torch.no_grad()
     def step(self, layer_idx: int = None, closure=None, *, clip_coef=None):
         """Update one layer (or all layers) from ``p.grad`` (layer_adam.py:271-359).
 
@@ -728,7 +675,6 @@ class LayerAdam:
         self._post_step(layer_idx)
         return loss
 
-    @torch.no_grad()
     def step_with_grad_views(self, layer_idx: int = None,
                              grad_views: Dict[torch.nn.Parameter, torch.Tensor] = None, closure=None, *,
                              clip_coef=None):
@@ -764,9 +710,12 @@ class LayerAdam:
         """Complete every host-tensor update still in flight (they are only in
         flight with ``overlap_host_chunks=True``)."""
         if self.overlap_host_chunks:
-            for streamer in self._streamers.values():
-                with torch.cuda.device(streamer.device):
-                    streamer.sync()
+            self._synchronize_streamers()
+
+    def _synchronize_streamers(self):
+        for streamer in self._streamers.values():
+            with torch.cuda.device(streamer.device):
+                streamer.sync()
 
     def _update_tensors(self, param_group, entries, clip_coef=None):
         """The per-tensor adam_update calls of step(layer) / step_with_grad_views
@@ -779,25 +728,30 @@ class LayerAdam:
         beta1, beta2 = param_group['betas']
         hp = (param_group['step'], param_group['lr'], beta1, beta2, param_group['eps'],
               param_group['weight_decay'], param_group['bias_correction'])
-        segs = _segments(entries) if len(entries) > 1 else None
-        if segs is not None and clip_coef is not None:
-            p0 = entries[0][0]
-            if (clip_coef.dtype != torch.float32 or clip_coef.numel() < 1 or not clip_coef.is_cuda
-                    or clip_coef.get_device() != p0.get_device()):
-                segs = None                  # the per-call path raises the reference-style error
-        if segs is not None:
-            p0, g0, m0, _ = entries[0]
-            with _on_device(p0.device):
-                rc = self.lib.la_adam_update_multi(
-                    self.optimizer_id, int(hp[0]), hp[1], hp[2], hp[3], hp[4], hp[5], int(bool(hp[6])),
-                    _DTYPE_CODE[p0.dtype], _DTYPE_CODE[g0.dtype], _DTYPE_CODE[m0.dtype], segs, len(entries),
-                    _ptr(clip_coef), _stream_handle(None, p0.device))
-            _lib.check(rc, "la_adam_update_multi")
-            return
-        for p, g, m, v in entries:
-            self.adam_update(*hp, p, g, m, v, clip_coef=clip_coef)
+        if len(entries) > 1:
+            index = entries[0][0].get_device()
+            if index >= 0:
+                device = entries[0][0].device
+                with _on_device(device):
+                    rc = self._host.update_multi(self.optimizer_id, int(hp[0]), hp[1], hp[2], hp[3], hp[4], hp[5],
+                                                 hp[6], index, _stream_handle(None, device), entries, clip_coef)
+                if rc is not None:
+                    _lib.check(rc, "la_adam_update_multi")
+                    return
+        # Host tensors: the calls are queued one behind the other on the link, and
+        # the last of them that has elements waits for all.
+        last = max((i for i, e in enumerate(entries) if not e[0].is_cuda and e[0].numel()), default=-1)
+        try:
+            for i, (p, g, m, v) in enumerate(entries):
+                if p.is_cuda:
+                    self.adam_update(*hp, p, g, m, v, clip_coef=clip_coef)
+                else:
+                    self._checked_update(*hp, p, g, m, v, None, clip_coef, None,
+                                         i == last and not self.overlap_host_chunks)
+        except BaseException:
+            self._synchronize_streamers()
+            raise
 
-    @torch.no_grad()
     def begin_chunk_step(self, layer_idx: int):
         """Start a chunked step: step += 1, NVMe prefetch (layer_adam.py:431-439)."""
         param_group = self.param_groups[layer_idx]
@@ -805,7 +759,6 @@ class LayerAdam:
         self._pre_step(layer_idx)
         return param_group
 
-    @torch.no_grad()
     def step_chunk(self, param_flat, grad_flat, exp_avg_flat, exp_avg_sq_flat, param_group, *,
                    bf16_out=None, clip_coef=None, stream=None):
         """Update one [cs:ce] chunk of flat tensors (layer_adam.py:442-461).
@@ -822,7 +775,6 @@ class LayerAdam:
                          param_group['bias_correction'], param_flat, grad_flat, exp_avg_flat,
                          exp_avg_sq_flat, bf16_out=bf16_out, clip_coef=clip_coef, stream=stream)
 
-    @torch.no_grad()
     def end_chunk_step(self, layer_idx: int):
         """End a chunked step: every chunk complete, then NVMe write-back (layer_adam.py:464-468)."""
         self.synchronize()
@@ -837,7 +789,6 @@ class LayerAdam:
     # ------------------------------------------------------------------
     # grad-norm clip (new; the reference has no clipping)
     # ------------------------------------------------------------------
-    @torch.no_grad()
     def clip_grad_norm(self, grads: Sequence[torch.Tensor], max_norm: float, *, stream=None):
         """Global L2 norm of device grads and the clip coefficient, both on device.
 
@@ -857,22 +808,23 @@ class LayerAdam:
         _check_grads(grads, device)
         nwork = _norm_workspace_elems(self.lib)
         with _on_device(device):
-            s = _torch_stream(stream, device)
-            handle = s.cuda_stream
+            handle = _stream_handle(stream, device)
             # scratch of this call only, one allocation on the stream it is used
-            # on, so calls on different streams share nothing: the partials,
-            # the float64 sum, then coef and norm as two fp32 in one more slot
+            # on, so calls on different streams share nothing: the partials and
+            # the float64 sum, then coef and norm, as fp32 elements
+            elems = 2 * (nwork + 1) + 2
             if stream is None:
-                buf = torch.empty(nwork + 2, dtype=torch.float64, device=device)
+                buf = torch.empty(elems, dtype=torch.float32, device=device)
             else:
-                with torch.cuda.stream(s):
-                    buf = torch.empty(nwork + 2, dtype=torch.float64, device=device)
+                with torch.cuda.stream(_torch_stream(stream, device)):
+                    buf = torch.empty(elems, dtype=torch.float32, device=device)
             base = buf.data_ptr()
-            work, sqnorm, cn = base, base + nwork * 8, base + (nwork + 1) * 8
-            pair = buf[nwork + 1:].view(torch.float32)
-            coef, norm = pair[0:1], pair[1:2]
+            sqnorm = base + nwork * 8
             # the first run of buffers overwrites the sum, the last one writes the coefficient
-            _norm_runs(self.lib, grads, work, nwork, sqnorm, False, float(max_norm), cn, handle)
+            rc = self._host.norm(grads, base, nwork * 8, sqnorm, False, float(max_norm), sqnorm + 8, handle)
+            if rc:
+                _lib.check(rc, "la_grad_sqnorm")
+            coef, norm = buf[-2:].split(1)
         return coef, norm
 
     def grad_norm_begin(self, device=None) -> "GradNormAccumulator":
@@ -906,8 +858,9 @@ class GradNormAccumulator:
         self.sqnorm = torch.zeros(1, dtype=torch.float64, device=self.device)
         self.work = torch.empty(_norm_workspace_elems(self.lib), dtype=torch.float64, device=self.device)
         self.count = 0
+        # the scratch belongs to the stream it was allocated on
+        self._home = _stream_handle(None, self.device)
 
-    @torch.no_grad()
     def add(self, grad, *, stream=None) -> None:
         """Add one grad buffer, or a sequence of them (a layer's per-tensor
         grads: two launches for up to 32 tensors of one dtype)."""
@@ -916,24 +869,30 @@ class GradNormAccumulator:
             return
         _check_grads(grads, self.device)
         with _on_device(self.device):
-            s = _torch_stream(stream, self.device)
-            _norm_runs(self.lib, grads, _ptr(self.work), self.work.numel(), _ptr(self.sqnorm), self.count > 0,
-                       0.0, None, s.cuda_stream)
-            self.work.record_stream(s)
-            self.sqnorm.record_stream(s)
+            handle = _stream_handle(stream, self.device)
+            rc = _lib.host_calls().norm(grads, self.work.data_ptr(), self.work.numel() * 8, self.sqnorm.data_ptr(),
+                                        self.count > 0, 0.0, 0, handle)
+            _lib.check(rc, "la_grad_norm_multi" if len(grads) > 1 else "la_grad_sqnorm")
+            self._record(stream, handle)
         self.count += 1
 
-    @torch.no_grad()
     def finish(self, max_norm: float, *, stream=None):
         """``(coef, norm)`` as fp32 device scalars, allocated on the stream that
         writes them; no host synchronisation."""
-        with torch.cuda.device(self.device):
-            s = _torch_stream(stream, self.device)
-            with torch.cuda.stream(s):
+        with _on_device(self.device):
+            handle = _stream_handle(stream, self.device)
+            with contextlib.nullcontext() if stream is None else torch.cuda.stream(_torch_stream(stream, self.device)):
                 coef = torch.empty(1, dtype=torch.float32, device=self.device)
                 norm = torch.empty(1, dtype=torch.float32, device=self.device)
             # with nothing added, sqnorm is still the zero it was created as: coef = 1
-            _lib.check(self.lib.la_clip_coef(_ptr(self.sqnorm), float(max_norm), _ptr(coef), _ptr(norm),
-                                             s.cuda_stream), "la_clip_coef")
-            self.sqnorm.record_stream(s)
+            _lib.check(self.lib.la_clip_coef(_ptr(self.sqnorm), float(max_norm), _ptr(coef), _ptr(norm), handle),
+                       "la_clip_coef")
+            self._record(stream, handle)
         return coef, norm
+
+    def _record(self, stream, handle) -> None:
+        """Mark the scratch as used by the stream of a launch, unless it is its own."""
+        if handle != self._home:
+            s = _torch_stream(stream, self.device)
+            self.work.record_stream(s)
+            self.sqnorm.record_stream(s)

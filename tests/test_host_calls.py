@@ -1,0 +1,50 @@
+"""The native host module on tensors it must leave to the per-call path, and its
+checks of grads.  No kernel is launched here."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from slideformer_amd import LayerAdam, _lib
+
+CALL = (1 << 19, 1, 1e-3, 0.9, 0.999, 1e-8, 0.01, True, 0, 0)    # an id that no test creates: a library call would fail
+
+
+def _cpu(n=8, dtype=torch.float32):
+    return torch.zeros(n, dtype=dtype)
+
+
+def test_update_leaves_host_tensors_and_other_objects_to_the_caller():
+    h = _lib.host_calls()
+    p, g, m, v = _cpu(), _cpu(), _cpu(), _cpu()
+    assert h.update(*CALL, p, g, m, v, None, None) is None
+    assert h.update(*CALL, torch.nn.Parameter(p), g, m, v, _cpu(dtype=torch.bfloat16), _cpu(1)) is None
+    assert h.update(*CALL, torch.empty(8, device="meta"), g, m, v, None, None) is None
+    assert h.update(*CALL, "p", g, m, v, None, None) is None
+    assert h.update(*CALL[:2], torch.tensor(1e-3), *CALL[3:], p, g, m, v, None, None) is None   # lr not a number
+    assert h.update_multi(*CALL, [(p, g, m, v)] * 2, None) is None
+    assert h.update_multi(*CALL, [], None) is None
+    assert h.update_multi(*CALL, [(p, g, m)], None) is None
+    with pytest.raises(TypeError):
+        h.update(*CALL, p)
+    with pytest.raises(TypeError):
+        h.update_multi(*CALL, ((p, g, m, v),), None)
+
+
+def test_check_grads_names_the_first_refused_grad():
+    h = _lib.host_calls()
+    assert h.check_grads([], 0) is None
+    assert h.check_grads([_cpu()], 0) == (0, 0)
+    with pytest.raises(TypeError):
+        h.check_grads([None], 0)
+
+
+def test_a_host_tensor_is_refused_without_a_device_and_the_scalars_have_advanced():
+    if torch.cuda.is_available():
+        pytest.skip("needs a machine without a HIP device")
+    adam = LayerAdam(lr=1e-3)
+    adam.add_layer_params(0, [torch.nn.Parameter(_cpu()), torch.nn.Parameter(_cpu())])
+    for q in adam.param_groups[0]["params"]:
+        q.grad = _cpu()
+    with pytest.raises(RuntimeError, match="HIP device"):
+        adam.step(0)
