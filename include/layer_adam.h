@@ -142,7 +142,8 @@ int la_adam_update_multi(int id, uint64_t step, float lr, float beta1, float bet
  * Grad norm (no counterpart in the reference, which has no clipping;
  * SlideFormer's update sits at transformer_layer.py:453-493): sum of squares
  * of g[0..n) in float64 into *sqnorm (device), added to the old value when
- * accumulate != 0.  Two kernels on `stream`: per-workgroup partials, then one
+ * accumulate != 0.  Two kernels on `stream` (one up to 131,072 elements):
+ * per-workgroup partials, then one
  * workgroup folds them.
  * `workspace` is caller-owned device memory of at least
  * la_grad_sqnorm_workspace(n) bytes, 8-byte aligned, holding the partials.
