@@ -739,7 +739,9 @@ class LayerAdam:
                     _lib.check(rc, "la_adam_update_multi")
                     return
         # Host tensors: the calls are queued one behind the other on the link, and
-        # the last of them that has elements waits for all.
+        # the last of them that has elements waits for all of its device; where
+        # grads or moments on several devices brought up several streamers, all
+        # of those are waited for.
         last = max((i for i, e in enumerate(entries) if not e[0].is_cuda and e[0].numel()), default=-1)
         try:
             for i, (p, g, m, v) in enumerate(entries):
@@ -748,6 +750,8 @@ class LayerAdam:
                 else:
                     self._checked_update(*hp, p, g, m, v, None, clip_coef, None,
                                          i == last and not self.overlap_host_chunks)
+            if last >= 0 and not self.overlap_host_chunks and len(self._streamers) > 1:
+                self._synchronize_streamers()
         except BaseException:
             self._synchronize_streamers()
             raise

@@ -48,3 +48,28 @@ def test_a_host_tensor_is_refused_without_a_device_and_the_scalars_have_advanced
         q.grad = _cpu()
     with pytest.raises(RuntimeError, match="HIP device"):
         adam.step(0)
+
+
+@pytest.mark.parametrize("overlap", [False, True])
+@pytest.mark.parametrize("streamers", [1, 2])
+def test_a_step_over_host_tensors_waits_for_every_streamer(streamers, overlap):
+    """The last call waits for its own device's streamer; a second one (grads on another device) is waited for too."""
+    calls = []
+
+    class Queued(LayerAdam):
+        def __init__(self):
+            self.overlap_host_chunks = overlap
+            self._streamers = dict.fromkeys(range(streamers))
+
+        def _checked_update(self, *args):
+            calls.append(args[-1])
+
+        def _synchronize_streamers(self):
+            calls.append("all")
+
+    entries = [(_cpu(), _cpu(), _cpu(), _cpu()) for _ in range(3)] + [(_cpu(0),) * 4]
+    group = {"step": 1, "lr": 1e-3, "betas": (0.9, 0.999), "eps": 1e-8, "weight_decay": 0.0, "bias_correction": True}
+    adam = Queued()     # kept: its end synchronizes once more
+    adam._update_tensors(group, entries)
+    waits = [False, False, not overlap, False]
+    assert calls == waits + (["all"] if streamers > 1 and not overlap else [])
