@@ -112,3 +112,68 @@ def test_norms_of_more_runs_than_one_launch_numbers(hip_device):
         assert abs(got - exact) <= 1e-12 * exact
         coef, norm = O.clip_coef(got, 0.5)
         assert cn[0].item() == np.float32(coef) and cn[1].item() == np.float32(norm)
+
+
+def test_gathered_norm_reads_changes_and_second_finish(hip_device):
+    """The accumulator's partials over calls of one and of many workgroups and of
+    several dtypes: a sum read between two adds, one changed in place (as an
+    all-reduce over ranks does) before finish, more adds after a finish."""
+    from slideformer_amd import LayerAdam
+
+    def make(n, kind):
+        return (torch.randn(n + 1, device=hip_device) * 1e-2).to(H.TD[kind])[1:]
+
+    def exact(grads):
+        return sum(O.grad_sqnorm(_bits(g, k), None if k == "f32" else k) for g, k in grads if g.numel())
+
+    acc = LayerAdam().grad_norm_begin(hip_device)
+    assert acc.sqnorm.item() == 0.0
+    grads = [(make(n, k), k) for n, k in [(ONE, "bf16"), (ONE + 1, "f32"), (0, "bf16"), (2_000_003, "f16"), (5, "f32")]]
+    acc.add(grads[0][0])
+    acc.add([g for g, _ in grads[1:]])
+    want = exact(grads)
+    for _ in range(2):
+        assert abs(acc.sqnorm.item() - want) <= 1e-12 * want
+    acc.sqnorm.mul_(4.0)
+    for more in ([], [(make(700_001, "bf16"), "bf16"), (make(9, "bf16"), "bf16")]):
+        before = exact(grads) * 4.0
+        for g, _ in more:
+            acc.add(g)
+        coef, norm = acc.finish(0.5)
+        want = before + exact(more)
+        got = acc.sqnorm.item()
+        print(f"gathered norm, {len(more)} more", flush=True)
+        assert abs(got - want) <= 1e-12 * want
+        c_ref, n_ref = O.clip_coef(got, 0.5)
+        assert coef.item() == np.float32(c_ref) and norm.item() == np.float32(n_ref)
+
+
+def test_gathered_norm_in_a_replayed_graph(hip_device):
+    """add, add, finish captured on an accumulator made before: every replay is the norm of the grads of its time."""
+    from slideformer_amd import LayerAdam
+
+    a, b = (torch.zeros(n, device=hip_device, dtype=torch.bfloat16) for n in (1_000_003, 77))
+    adam = LayerAdam()
+    warm, acc = adam.grad_norm_begin(hip_device), adam.grad_norm_begin(hip_device)
+    warm.add(a)
+    warm.add([b, a])
+    warm.finish(1.0)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        acc.add(a)
+        acc.add([b, a])
+        coef, norm = acc.finish(1.0)
+    for replay, scale in enumerate((1e-2, 1.0, 1e-3)):
+        for t in (a, b):
+            t.copy_(torch.randn(t.numel(), device=hip_device) * scale)
+        graph.replay()
+        torch.cuda.synchronize()
+        if replay:              # the sum that the replay left, finished outside the graph
+            eager = acc.finish(1.0)
+            assert torch.equal(eager[0], coef) and torch.equal(eager[1], norm)
+        sq = 2 * O.grad_sqnorm(_bits(a, "bf16"), "bf16") + O.grad_sqnorm(_bits(b, "bf16"), "bf16")
+        print(f"gathered norm replay, scale {scale}", flush=True)
+        # the float64 sum is within 1e-12, so the fp32 norm is within one rounding of its last place
+        assert abs(norm.item() - sq ** 0.5) <= 2.0 ** -23 * sq ** 0.5
+        assert coef.item() == np.float32(O.clip_coef(float(norm.item()) ** 2, 1.0)[0])
