@@ -189,24 +189,6 @@ int la_grad_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, voi
                        float* coef, float* norm_out, la_stream_t stream);
 
 /*
- * A norm gathered over many calls (a global clip over layers that pass one by
- * one), one launch per call: la_grad_norm_add adds the sum of squares of
- * bufs[0..count), as la_grad_norm_multi takes them, to float64 partials;
- * with accumulate == 0 it starts a new sum in them and clears *sqnorm.
- * la_grad_norm_fold adds the partials to *sqnorm, leaves zeros in them and, with
- * coef != NULL, writes the clip coefficient of *sqnorm (and *norm_out when not
- * NULL), as la_clip_coef computes it; folded again, the result is the same.
- * `partials`: device memory, 8-byte aligned, of the same partials_bytes in every
- * call, at least la_grad_sqnorm_workspace(N) bytes for N the elements of the
- * largest call, at most LA_NORM_SCRATCH_PARTIALS * 8.  Calls on the same
- * partials must be ordered.
- */
-int la_grad_norm_add(int g_dtype, const la_grad_buffer_t* bufs, int count, void* partials,
-                     uint64_t partials_bytes, double* sqnorm, int accumulate, la_stream_t stream);
-int la_grad_norm_fold(void* partials, uint64_t partials_bytes, double* sqnorm, float max_norm,
-                      float* coef, float* norm_out, la_stream_t stream);
-
-/*
  * la_grad_norm_clip without a workspace: for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  No counterpart in the reference.  The stage-1

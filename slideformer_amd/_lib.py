@@ -58,8 +58,6 @@ EXPORTED = (
     "la_grad_sqnorm",
     "la_grad_norm_clip",
     "la_grad_norm_multi",
-    "la_grad_norm_add",
-    "la_grad_norm_fold",
     "la_grad_norm_clip_noalloc",
     "la_clip_coef",
     "la_pipeline_workspace_bytes",
@@ -169,10 +167,6 @@ def _declare(L):
     L.la_grad_norm_clip.restype = i
     L.la_grad_norm_multi.argtypes = [i, ctypes.POINTER(LaGradBuffer), i, P, u64, P, i, f, P, P, P]
     L.la_grad_norm_multi.restype = i
-    L.la_grad_norm_add.argtypes = [i, ctypes.POINTER(LaGradBuffer), i, P, u64, P, i, P]
-    L.la_grad_norm_add.restype = i
-    L.la_grad_norm_fold.argtypes = [P, u64, P, f, P, P, P]
-    L.la_grad_norm_fold.restype = i
     L.la_grad_norm_clip_noalloc.argtypes = [i, P, u64, P, i, f, P, P, P]
     L.la_grad_norm_clip_noalloc.restype = i
     L.la_clip_coef.argtypes = [P, f, P, P, P]
@@ -247,7 +241,7 @@ def host_calls():
                 spec.loader.exec_module(module)
                 module.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
                     L.la_adam_update, L.la_adam_update_multi, L.la_grad_sqnorm, L.la_grad_norm_clip,
-                    L.la_grad_norm_multi, L.la_grad_norm_add)))
+                    L.la_grad_norm_multi)))
                 _host_calls = module
     return _host_calls
 

@@ -32,7 +32,6 @@ decltype(&la_adam_update_multi) p_update_multi = nullptr;
 decltype(&la_grad_sqnorm) p_sqnorm = nullptr;
 decltype(&la_grad_norm_clip) p_norm_clip = nullptr;
 decltype(&la_grad_norm_multi) p_norm_multi = nullptr;
-decltype(&la_grad_norm_add) p_norm_add = nullptr;
 
 int code_of(const at::Tensor& t)
 {
@@ -230,15 +229,14 @@ try {
     return failed(e.what());
 }
 
-// norm(grads, workspace, its bytes, sqnorm, accumulate, max_norm, cn | 0 | None, stream) -> rc
+// norm(grads, workspace, its bytes, sqnorm, accumulate, max_norm, cn | 0, stream) -> rc
 // The sum of squares of checked grads into the float64 at `sqnorm` (added to
 // it when accumulate): runs of one dtype, at most LA_NORM_MULTI_MAX buffers
 // each, one library call per run, later runs adding to the earlier ones;
 // la_grad_norm_multi for a run of several buffers, la_grad_sqnorm /
 // la_grad_norm_clip for a run of one (the same bits, a smaller launch).  With
 // `cn` (address of two fp32: coef, norm) the last call also writes the clip
-// coefficient.  With `cn` None the sums stay in the workspace's partials
-// (la_grad_norm_add).
+// coefficient.
 PyObject* norm(PyObject*, PyObject* const* a, Py_ssize_t n)
 try {
     if (n != 8 || !PyList_Check(a[0])) return PyErr_Format(PyExc_TypeError, "norm takes a list and 7 arguments");
@@ -247,8 +245,7 @@ try {
     double* sqnorm = static_cast<double*>(PyLong_AsVoidPtr(a[3]));
     const int accumulate = PyObject_IsTrue(a[4]);
     const float max_norm = static_cast<float>(PyFloat_AsDouble(a[5]));
-    const bool keep = a[6] == Py_None;
-    float* cn = keep ? nullptr : static_cast<float*>(PyLong_AsVoidPtr(a[6]));
+    float* cn = static_cast<float*>(PyLong_AsVoidPtr(a[6]));
     const la_stream_t stream = PyLong_AsVoidPtr(a[7]);
     if (PyErr_Occurred()) return nullptr;
     const Py_ssize_t count = PyList_GET_SIZE(a[0]);
@@ -266,9 +263,7 @@ try {
         while (end < count && codes[end] == codes[k] && end - k < LA_NORM_MULTI_MAX) ++end;
         float* coef = end == count ? cn : nullptr;
         const int acc = accumulate || k > 0;
-        if (keep)
-            rc = p_norm_add(codes[k], &bufs[k], static_cast<int>(end - k), work, bytes, sqnorm, acc, stream);
-        else if (end - k > 1)
+        if (end - k > 1)
             rc = p_norm_multi(codes[k], &bufs[k], static_cast<int>(end - k), work, bytes, sqnorm, acc, max_norm, coef,
                               coef ? coef + 1 : nullptr, stream);
         else if (coef)
@@ -284,12 +279,12 @@ try {
 }
 
 // bind(addresses of la_adam_update, la_adam_update_multi, la_grad_sqnorm,
-// la_grad_norm_clip, la_grad_norm_multi, la_grad_norm_add): of the library _lib has loaded.
+// la_grad_norm_clip, la_grad_norm_multi): of the library _lib has loaded.
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    if (n != 6) return PyErr_Format(PyExc_TypeError, "bind takes 6 addresses");
-    void* at[6];
-    for (int k = 0; k < 6; ++k) {
+    if (n != 5) return PyErr_Format(PyExc_TypeError, "bind takes 5 addresses");
+    void* at[5];
+    for (int k = 0; k < 5; ++k) {
         at[k] = PyLong_AsVoidPtr(a[k]);
         if (!at[k]) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_ValueError, "bind: null address");
     }
@@ -298,7 +293,6 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n)
     p_sqnorm = reinterpret_cast<decltype(p_sqnorm)>(at[2]);
     p_norm_clip = reinterpret_cast<decltype(p_norm_clip)>(at[3]);
     p_norm_multi = reinterpret_cast<decltype(p_norm_multi)>(at[4]);
-    p_norm_add = reinterpret_cast<decltype(p_norm_add)>(at[5]);
     Py_RETURN_NONE;
 }
 

@@ -26,8 +26,7 @@
 // LDS, and writes one partial per workgroup to the caller's workspace; stage 2
 // (one workgroup) folds the partials in a fixed order and, optionally, writes
 // the clip coefficient.  Up to LA_NORM_ONE elements stage 1 is one workgroup
-// and ends the call itself.  A norm gathered over calls is one launch each, the
-// partials adding up in their slots until la_grad_norm_fold.
+// and ends the call itself.
 
 #include <hip/hip_runtime.h>
 
@@ -545,7 +544,6 @@ struct NormArgs {
     float max_norm;
     float* coef;          // may be null: then only *sqnorm is written
     float* norm_out;      // may be null
-    uint32_t slots;       // not 0: the sum stays in this many partials (la_grad_norm_add)
 };
 
 // The total of a norm call, in one thread.
@@ -557,19 +555,11 @@ __device__ __forceinline__ void write_norm(const NormArgs& a, double total)
 }
 
 // End of stage 1: the workgroup's partial, or, on a grid of one workgroup, the
-// call's result.  Of a sum that stays in the partials every slot has one writer
-// per launch; its first call (accumulate 0) overwrites them all and clears *sqnorm.
-// Measured on MI355X, the clipped step of 13 layers of 7.1-39 M elements, norms
-// layer by layer: 655 us with a fold behind every layer's stage 1, 637 with one.
+// call's result.
 __device__ __forceinline__ void sqnorm_end(const NormArgs& a, double t)
 {
-    if (a.slots && !a.accumulate && blockIdx.x == 0)
-        for (uint32_t i = gridDim.x + threadIdx.x; i < a.slots; i += LA_NORM_BLOCK) a.partials[i] = 0.0;
     if (threadIdx.x != 0) return;
-    if (a.slots) {
-        a.partials[blockIdx.x] = a.accumulate ? a.partials[blockIdx.x] + t : t;
-        if (!a.accumulate && blockIdx.x == 0) *a.sqnorm = 0.0;
-    } else if (gridDim.x == 1) write_norm(a, t);
+    if (gridDim.x == 1) write_norm(a, t);
     else a.partials[blockIdx.x] = t;
 }
 
@@ -683,16 +673,11 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N>
 // Stage 2, one workgroup: fold the stage-1 partials in a fixed order.  The
 // kernel boundary makes every partial visible: a single-launch "last
 // workgroup" fold would need an agent-scope release per workgroup, which on
-// gfx950 writes back the whole per-XCD L2 each time.  With TAKE (partials that
-// several calls added to) it leaves zeros behind.
-template <bool TAKE>
+// gfx950 writes back the whole per-XCD L2 each time.
 __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_finish(NormArgs a, uint32_t nparts)
 {
     double s = 0.0;
-    for (uint32_t i = threadIdx.x; i < nparts; i += LA_NORM_BLOCK) {
-        s += a.partials[i];
-        if (TAKE) a.partials[i] = 0.0;
-    }
+    for (uint32_t i = threadIdx.x; i < nparts; i += LA_NORM_BLOCK) s += a.partials[i];
     const double total = block_sum_f64(s);
     if (threadIdx.x == 0) write_norm(a, total);
 }
@@ -1012,7 +997,7 @@ void derive_scalars(HostState& s, uint64_t step, float lr, float b1, float b2, f
 }
 
 // Stage 1 over `count` <= N checked buffers on `grid` workgroups, and the fold
-// of its partials where they are more than one and the call has a sum to write.
+// of its partials where they are more than one.
 template <int N>
 int launch_sqnorm(int g_dtype, const la_grad_buffer_t* bufs, int count, uint32_t grid, const NormArgs& end,
                   hipStream_t st)
@@ -1043,14 +1028,12 @@ int launch_sqnorm(int g_dtype, const la_grad_buffer_t* bufs, int count, uint32_t
                       dim3(LA_NORM_BLOCK), 0, st, m);
     };
     const int rc = g_dtype == LA_F32 ? stage1(float{}) : g_dtype == LA_BF16 ? stage1(bf16_t{}) : stage1(f16_t{});
-    if (rc != LA_OK || grid == 1 || end.slots) return rc;
-    return launch(la_sqnorm_finish<false>, dim3(1), dim3(LA_NORM_BLOCK), 0, st, end, grid);
+    if (rc != LA_OK || grid == 1) return rc;
+    return launch(la_sqnorm_finish, dim3(1), dim3(LA_NORM_BLOCK), 0, st, end, grid);
 }
 
-// `keep`: the sum stays in the workspace, all of its slots.
 int launch_norm(int g_dtype, const void* g, uint64_t n, void* workspace, uint64_t workspace_bytes,
-                double* sqnorm, int accumulate, float max_norm, float* coef, float* norm_out, hipStream_t st,
-                bool keep = false)
+                double* sqnorm, int accumulate, float max_norm, float* coef, float* norm_out, hipStream_t st)
 {
     if (!dt_valid(g_dtype)) return LA_EDTYPE;
     if (!sqnorm || !workspace) return LA_EINVAL;
@@ -1069,20 +1052,19 @@ int launch_norm(int g_dtype, const void* g, uint64_t n, void* workspace, uint64_
         // more runs than the kernel's 32-bit run numbers hold: part by part
         const uint64_t half = n / 2 / kVec * kVec;
         const int rc = launch_norm(g_dtype, g, half, workspace, workspace_bytes, sqnorm, accumulate, max_norm, nullptr,
-                                   nullptr, st, keep);
+                                   nullptr, st);
         if (rc != LA_OK) return rc;
         return launch_norm(g_dtype, static_cast<const char*>(g) + half * gb, n - half, workspace, workspace_bytes,
-                           sqnorm, 1, max_norm, coef, norm_out, st, keep);
+                           sqnorm, 1, max_norm, coef, norm_out, st);
     }
     const la_grad_buffer_t buf{g, n};
-    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out,
-                       keep ? static_cast<uint32_t>(workspace_bytes / sizeof(double)) : 0};
+    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out};
     return launch_sqnorm<1>(g_dtype, &buf, 1, norm_grid(n), end, st);
 }
 
 int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void* workspace,
                       uint64_t workspace_bytes, double* sqnorm, int accumulate, float max_norm, float* coef,
-                      float* norm_out, hipStream_t st, bool keep = false)
+                      float* norm_out, hipStream_t st)
 {
     if (!dt_valid(g_dtype)) return LA_EDTYPE;
     if (!bufs || count < 1 || count > LA_NORM_MULTI_MAX || !sqnorm || !workspace) return LA_EINVAL;
@@ -1112,13 +1094,12 @@ int launch_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, void
             const bool final = b + 1 == count;
             const int rc = launch_norm(g_dtype, bufs[b].g, bufs[b].n, workspace, workspace_bytes, sqnorm,
                                        accumulate || b > 0, max_norm, final ? coef : nullptr,
-                                       final ? norm_out : nullptr, st, keep);
+                                       final ? norm_out : nullptr, st);
             if (rc != LA_OK) return rc;
         }
         return LA_OK;
     }
-    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out,
-                       keep ? static_cast<uint32_t>(workspace_bytes / sizeof(double)) : 0};
+    const NormArgs end{static_cast<double*>(workspace), sqnorm, accumulate ? 1 : 0, max_norm, coef, norm_out};
     return launch_sqnorm<LA_NORM_MULTI_MAX>(g_dtype, bufs, count, norm_grid(total), end, st);
 }
 
@@ -1376,35 +1357,6 @@ int la_grad_norm_multi(int g_dtype, const la_grad_buffer_t* bufs, int count, voi
 {
     return launch_norm_multi(g_dtype, bufs, count, workspace, workspace_bytes, sqnorm, accumulate, max_norm, coef,
                              norm_out, static_cast<hipStream_t>(stream));
-}
-
-int la_grad_norm_add(int g_dtype, const la_grad_buffer_t* bufs, int count, void* partials, uint64_t partials_bytes,
-                     double* sqnorm, int accumulate, la_stream_t stream)
-{
-    if (partials_bytes % sizeof(double) || partials_bytes > LA_NORM_SCRATCH_PARTIALS * sizeof(double))
-        return LA_EINVAL;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (bufs && count == 1)
-        return launch_norm(g_dtype, bufs->g, bufs->n, partials, partials_bytes, sqnorm, accumulate, 0.0f, nullptr,
-                           nullptr, st, true);
-    return launch_norm_multi(g_dtype, bufs, count, partials, partials_bytes, sqnorm, accumulate, 0.0f, nullptr,
-                             nullptr, st, true);
-}
-
-int la_grad_norm_fold(void* partials, uint64_t partials_bytes, double* sqnorm, float max_norm, float* coef,
-                      float* norm_out, la_stream_t stream)
-{
-    if (!partials || !sqnorm || partials_bytes == 0 || partials_bytes % sizeof(double) ||
-        partials_bytes > LA_NORM_SCRATCH_PARTIALS * sizeof(double))
-        return LA_EINVAL;
-    if ((reinterpret_cast<uintptr_t>(sqnorm) & 7u) || (reinterpret_cast<uintptr_t>(partials) & 7u)) return LA_EINVAL;
-    if ((reinterpret_cast<uintptr_t>(coef) & 3u) || (reinterpret_cast<uintptr_t>(norm_out) & 3u)) return LA_EINVAL;
-    if (!device_accessible(partials) || !device_accessible(sqnorm) || (coef && !device_accessible(coef)) ||
-        (norm_out && !device_accessible(norm_out)))
-        return LA_EFAULT;
-    const NormArgs end{static_cast<double*>(partials), sqnorm, 1, max_norm, coef, norm_out, 0};
-    return launch(la_sqnorm_finish<true>, dim3(1), dim3(LA_NORM_BLOCK), 0, static_cast<hipStream_t>(stream), end,
-                  static_cast<uint32_t>(partials_bytes / sizeof(double)));
 }
 
 int la_grad_norm_clip_noalloc(int g_dtype, const void* g, uint64_t n, double* sqnorm, int accumulate,

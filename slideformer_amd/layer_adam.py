@@ -846,12 +846,15 @@ class LayerAdam:
 
 class GradNormAccumulator:
     """Float64 sum of squares accumulated over several device buffers
-    (la_grad_norm_add: one launch for each buffer, or for a list of them, into
-    running partials), then one clip coefficient (la_grad_norm_fold).
+    (la_grad_sqnorm, or la_grad_norm_multi for a list of them, with
+    accumulate), then one clip coefficient (la_clip_coef).
 
-    One accumulator is one running sum: its ``add`` and ``finish`` calls, and
-    reads of ``sqnorm``, must be ordered, i.e. on one stream or synchronised
-    between streams.  Its scratch
+    ``sqnorm``, one float64 on the device, is the running sum itself: each add
+    leaves it complete on that add's stream, and ``finish`` takes what it holds
+    (for instance after an all-reduce over ranks).
+
+    One accumulator is one running sum: its ``add`` and ``finish`` calls must be
+    ordered, i.e. on one stream or synchronised between streams.  Its scratch
     is allocated once, at the size any buffer needs, and is marked as used by
     every stream a launch runs on (``record_stream``), so that the caching
     allocator does not hand it out again before those launches are done, even
@@ -860,34 +863,24 @@ class GradNormAccumulator:
     def __init__(self, device):
         self.lib = _lib.load()
         self.device = torch.device(device)
-        nwork = _norm_workspace_elems(self.lib)
-        # the partials, and behind them the sum they are folded into
-        self._scratch = torch.zeros(nwork + 1, dtype=torch.float64, device=self.device)
-        self._work, self._bytes = self._scratch.data_ptr(), nwork * 8
+        self.sqnorm = torch.zeros(1, dtype=torch.float64, device=self.device)
+        self.work = torch.empty(_norm_workspace_elems(self.lib), dtype=torch.float64, device=self.device)
         self.count = 0
         # the scratch belongs to the stream it was allocated on
         self._home = _stream_handle(None, self.device)
 
-    @property
-    def sqnorm(self):
-        """The sum of squares so far, one float64 on the device (``finish`` takes what it holds, for instance
-        after an all-reduce over ranks)."""
-        with _on_device(self.device):
-            self._fold(0.0, None, None, None)
-        return self._scratch[-1:]
-
     def add(self, grad, *, stream=None) -> None:
         """Add one grad buffer, or a sequence of them (a layer's per-tensor
-        grads: one launch for up to 32 tensors of one dtype)."""
+        grads: two launches for up to 32 tensors of one dtype)."""
         grads = [grad] if isinstance(grad, torch.Tensor) else [g for g in grad if g is not None]
         if not grads:
             return
         _check_grads(grads, self.device)
         with _on_device(self.device):
             handle = _stream_handle(stream, self.device)
-            rc = _lib.host_calls().norm(grads, self._work, self._bytes, self._work + self._bytes, self.count > 0, 0.0,
-                                        None, handle)
-            _lib.check(rc, "la_grad_norm_add")
+            rc = _lib.host_calls().norm(grads, self.work.data_ptr(), self.work.numel() * 8, self.sqnorm.data_ptr(),
+                                        self.count > 0, 0.0, 0, handle)
+            _lib.check(rc, "la_grad_norm_multi" if len(grads) > 1 else "la_grad_sqnorm")
             self._record(stream, handle)
         self.count += 1
 
@@ -895,22 +888,19 @@ class GradNormAccumulator:
         """``(coef, norm)`` as fp32 device scalars, allocated on the stream that
         writes them; no host synchronisation."""
         with _on_device(self.device):
+            handle = _stream_handle(stream, self.device)
             with contextlib.nullcontext() if stream is None else torch.cuda.stream(_torch_stream(stream, self.device)):
                 coef = torch.empty(1, dtype=torch.float32, device=self.device)
                 norm = torch.empty(1, dtype=torch.float32, device=self.device)
-            # with nothing added, all is still the zeros it was created as: coef = 1
-            self._fold(float(max_norm), coef, norm, stream)
+            # with nothing added, sqnorm is still the zero it was created as: coef = 1
+            _lib.check(self.lib.la_clip_coef(_ptr(self.sqnorm), float(max_norm), _ptr(coef), _ptr(norm), handle),
+                       "la_clip_coef")
+            self._record(stream, handle)
         return coef, norm
-
-    def _fold(self, max_norm, coef, norm, stream) -> None:
-        # always a launch: replayed graphs add to the partials without this object's knowledge
-        handle = _stream_handle(stream, self.device)
-        _lib.check(self.lib.la_grad_norm_fold(self._work, self._bytes, self._work + self._bytes, max_norm, _ptr(coef),
-                                              _ptr(norm), handle), "la_grad_norm_fold")
-        self._record(stream, handle)
 
     def _record(self, stream, handle) -> None:
         """Mark the scratch as used by the stream of a launch, unless it is its own."""
         if handle != self._home:
             s = _torch_stream(stream, self.device)
-            self._scratch.record_stream(s)
+            self.work.record_stream(s)
+            self.sqnorm.record_stream(s)

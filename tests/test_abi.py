@@ -149,16 +149,6 @@ def test_error_codes_without_launch():
     bufs[1].n = 0                                                                         # empty: g may be NULL
     assert multi(1, bufs, 2, hp, 64, hp, 0, 1.0, hp, None, None) == _lib.LA_EFAULT
     assert multi(1, bufs, _lib.LA_NORM_MULTI_MAX, hp, 64, hp, 1, 0.0, None, None, None) == _lib.LA_EFAULT
-    # the gathered norm: as above; its fold takes whole partials, no more than a stage 1 writes
-    add, fold = L.la_grad_norm_add, L.la_grad_norm_fold
-    assert add(1, None, 1, hp, 64, hp, 0, None) == add(1, bufs, 0, hp, 64, hp, 0, None) == _lib.LA_EINVAL
-    for work, size, sq in ((None, 64, hp), (hp, 0, hp), (hp, 64, None), (hp + 4, 64, hp), (hp, 64, hp + 4),
-                           (hp, 12, hp), (hp, 257 * 8, hp)):
-        assert add(1, bufs, 1, work, size, sq, 1, None) == add(1, bufs, 2, work, size, sq, 0, None) == _lib.LA_EINVAL
-        assert fold(work, size, sq, 1.0, None, None, None) == _lib.LA_EINVAL
-    assert add(7, bufs, 1, hp, 64, hp, 0, None) == _lib.LA_EDTYPE
-    assert add(1, bufs, 1, hp, 64, hp, 0, None) == add(1, bufs, 2, hp, 64, hp, 0, None) == _lib.LA_EFAULT
-    assert fold(hp, 64, hp, 1.0, hp, hp, None) == _lib.LA_EFAULT
     assert b"device memory" in L.la_strerror(_lib.LA_EFAULT)
     assert b"dtype" in L.la_strerror(_lib.LA_EDTYPE)
     assert b"memory" in L.la_strerror(_lib.LA_ENOMEM)

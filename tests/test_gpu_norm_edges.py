@@ -177,3 +177,29 @@ def test_gathered_norm_in_a_replayed_graph(hip_device):
         # the float64 sum is within 1e-12, so the fp32 norm is within one rounding of its last place
         assert abs(norm.item() - sq ** 0.5) <= 2.0 ** -23 * sq ** 0.5
         assert coef.item() == np.float32(O.clip_coef(float(norm.item()) ** 2, 1.0)[0])
+
+
+def test_sqnorm_is_the_running_sum_itself(hip_device):
+    """acc.sqnorm is one tensor for the accumulator's life: taken before the adds it holds each of them as its
+    stream gets there, changed in place (an all-reduce over ranks) it is what finish takes, and reading the
+    attribute launches nothing, so it needs no order with adds that still run on another stream."""
+    from slideformer_amd import LayerAdam
+
+    grads = [(torch.randn(n, device=hip_device) * 1e-2).bfloat16() for n in (300_001, 5, ONE + 1)]
+    sums = [O.grad_sqnorm(_bits(g, "bf16"), "bf16") for g in grads]
+    acc = LayerAdam().grad_norm_begin(hip_device)
+    held = acc.sqnorm
+    torch.cuda.synchronize()
+    acc.add(grads[0])
+    assert abs(held.item() - sums[0]) <= 1e-12 * sums[0]
+    side = torch.cuda.Stream()
+    acc.add(grads[1:], stream=side)
+    assert acc.sqnorm is held
+    side.synchronize()
+    want = sum(sums)
+    assert abs(held.item() - want) <= 1e-12 * want
+    held.mul_(9.0)
+    coef, norm = acc.finish(0.25)
+    c_ref, n_ref = O.clip_coef(held.item(), 0.25)
+    assert abs(held.item() - 9.0 * want) <= 9e-12 * want
+    assert coef.item() == np.float32(c_ref) and norm.item() == np.float32(n_ref)
