@@ -143,6 +143,9 @@ struct la_pipeline {
     const char* last_ws = nullptr;
     uint64_t last_slot_bytes = 0;
     bool pending_direct = false;  // direct launches that no call has waited for yet
+    // a direct call that launches on its caller's stream, while it runs
+    bool on_caller = false;
+    hipStream_t caller = nullptr;
     uint64_t calls = 0;  // la_pipeline_step calls so far (the trace's call numbers)
 };
 
@@ -249,11 +252,13 @@ int enter_ring(la_pipeline* pl, bool direct, uint64_t slots, const char* base, u
     return LA_OK;
 }
 
-// After a failure part-way through a call, let the queued copies finish before
-// returning, so that nothing still writes the caller's memory afterwards, and
-// deliver the copy-outs of every chunk whose copy-back was queued.
+// After a failure part-way through a call, let the queued copies and launches
+// finish before returning, so that nothing still writes the caller's memory
+// afterwards, and deliver the copy-outs of every chunk whose copy-back was queued.
 int drain_streams(la_pipeline* pl, int rc)
 {
+    if (pl->on_caller) (void)hipStreamSynchronize(pl->caller);
+    pl->on_caller = false;
     (void)hipStreamSynchronize(pl->h2d);
     (void)hipStreamSynchronize(pl->comp);
     (void)hipStreamSynchronize(pl->d2h);
@@ -351,6 +356,8 @@ int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtyp
     // stream of its own.
     const bool own = !wait || staged || pl->pending_direct;
     hipStream_t st = own ? pl->comp : caller;
+    pl->on_caller = !own;
+    pl->caller = caller;
     LA_DIRECT_TRY(hipEventRecord(pl->t_begin, caller));
     if (staged) LA_DIRECT_TRY(hipEventSynchronize(pl->t_begin));
     else if (own) LA_DIRECT_TRY(hipStreamWaitEvent(st, pl->t_begin, 0));
@@ -412,6 +419,7 @@ int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtyp
     }
     LA_DIRECT_TRY(hipEventSynchronize(pl->t_end));
 #undef LA_DIRECT_TRY
+    pl->on_caller = false;
     pl->touched.clear();
     pl->pending_direct = false;
     if (stats) {
