@@ -95,7 +95,7 @@ bool parse(PyObject* const* a, Call& c)
     for (int k = 2; k < 7; ++k)
         if (!PyFloat_Check(a[k]) && !PyLong_Check(a[k])) return false;
     c.id = static_cast<int>(PyLong_AsLong(a[0]));
-    c.step = PyLong_AsUnsignedLongLong(a[1]);
+    c.step = PyLong_AsUnsignedLongLongMask(a[1]);    // modulo 2^64, as a ctypes uint64 argument takes it
     c.lr = static_cast<float>(PyFloat_AsDouble(a[2]));
     c.beta1 = static_cast<float>(PyFloat_AsDouble(a[3]));
     c.beta2 = static_cast<float>(PyFloat_AsDouble(a[4]));

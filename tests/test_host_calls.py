@@ -31,6 +31,14 @@ def test_update_leaves_host_tensors_and_other_objects_to_the_caller():
         h.update_multi(*CALL, ((p, g, m, v),), None)
 
 
+@pytest.mark.parametrize("step", [-1, 2 ** 64 + 7])
+def test_a_step_number_beyond_64_bits_wraps_as_in_the_per_call_path(step):
+    h = _lib.host_calls()
+    p, g, m, v = _cpu(), _cpu(), _cpu(), _cpu()
+    assert h.update(CALL[0], step, *CALL[2:], p, g, m, v, None, None) is None
+    assert h.update_multi(CALL[0], step, *CALL[2:], [(p, g, m, v)] * 2, None) is None
+
+
 def test_check_grads_names_the_first_refused_grad():
     h = _lib.host_calls()
     assert h.check_grads([], 0) is None
