@@ -88,19 +88,27 @@ struct Call {
 };
 constexpr Py_ssize_t kCallArgs = 10;
 
-// False with an exception set, or without one for a hyper-parameter that is
-// not a Python number (the caller's path then decides about it).
+// False with an exception set, or without one for a hyper-parameter that is no
+// number: anything with a float value is one, as for a ctypes float argument
+// (the caller's path then decides about it).
 bool parse(PyObject* const* a, Call& c)
 {
-    for (int k = 2; k < 7; ++k)
-        if (!PyFloat_Check(a[k]) && !PyLong_Check(a[k])) return false;
+    float x[5];
+    for (int k = 0; k < 5; ++k) {
+        const double d = PyFloat_AsDouble(a[2 + k]);
+        if (d == -1.0 && PyErr_Occurred()) {
+            PyErr_Clear();
+            return false;
+        }
+        x[k] = static_cast<float>(d);
+    }
     c.id = static_cast<int>(PyLong_AsLong(a[0]));
     c.step = PyLong_AsUnsignedLongLongMask(a[1]);    // modulo 2^64, as a ctypes uint64 argument takes it
-    c.lr = static_cast<float>(PyFloat_AsDouble(a[2]));
-    c.beta1 = static_cast<float>(PyFloat_AsDouble(a[3]));
-    c.beta2 = static_cast<float>(PyFloat_AsDouble(a[4]));
-    c.eps = static_cast<float>(PyFloat_AsDouble(a[5]));
-    c.wd = static_cast<float>(PyFloat_AsDouble(a[6]));
+    c.lr = x[0];
+    c.beta1 = x[1];
+    c.beta2 = x[2];
+    c.eps = x[3];
+    c.wd = x[4];
     c.bias_correction = PyObject_IsTrue(a[7]);
     c.dev = PyLong_AsLongLong(a[8]);
     c.stream = PyLong_AsVoidPtr(a[9]);

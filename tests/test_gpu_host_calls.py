@@ -74,6 +74,40 @@ def test_step_equals_one_call_per_tensor(form, hip_device):
         assert np.array_equal(a, b)
 
 
+class _Recorded:
+    """The native host module, with what its update_multi calls returned."""
+
+    def __init__(self, host):
+        self.host, self.returned = host, []
+
+    def __getattr__(self, name):
+        return getattr(self.host, name)
+
+    def update_multi(self, *args):
+        self.returned.append(self.host.update_multi(*args))
+        return self.returned[-1]
+
+
+def _step(dev, params, grads, coef=None, **group):
+    """One step(layer) of params with grads: what its batched call returned and every bit of the result."""
+    adam = LayerAdam(lr=1e-3, weight_decay=0.01)
+    adam._host = _Recorded(adam._host)
+    adam.add_layer_params(0, params)
+    adam.param_groups[0].update(group)
+    adam.step_with_grad_views(0, dict(zip(params, grads)), clip_coef=coef)
+    return adam._host.returned, [_bits(t) for t in (*params, adam.exp_avg_flat[0], adam.exp_avg_sq_flat[0])]
+
+
+@pytest.mark.parametrize("kind", ["np.float32", "tensor", "device tensor", "np array"])
+def test_hyper_parameters_of_any_number_type_keep_the_batched_launch(kind, hip_device):
+    lr = {"np.float32": np.float32(1e-3), "tensor": torch.tensor(1e-3), "np array": np.array(1e-3, np.float32),
+          "device tensor": torch.tensor(1e-3, device=hip_device)}[kind]
+    returned, got = _step(hip_device, *_layer(hip_device, torch.float32, 4), lr=lr, betas=(np.float32(0.9), 0.999))
+    assert returned == [0]
+    for a, b in zip(got, _step(hip_device, *_layer(hip_device, torch.float32, 4))[1]):
+        assert np.array_equal(a, b)
+
+
 def test_refused_calls_still_raise_and_complete_what_was_queued(hip_device):
     adam = LayerAdam(lr=1e-3)
     p, m, v = (torch.zeros(16, device=hip_device) for _ in range(3))

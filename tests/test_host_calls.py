@@ -21,7 +21,9 @@ def test_update_leaves_host_tensors_and_other_objects_to_the_caller():
     assert h.update(*CALL, torch.nn.Parameter(p), g, m, v, _cpu(dtype=torch.bfloat16), _cpu(1)) is None
     assert h.update(*CALL, torch.empty(8, device="meta"), g, m, v, None, None) is None
     assert h.update(*CALL, "p", g, m, v, None, None) is None
-    assert h.update(*CALL[:2], torch.tensor(1e-3), *CALL[3:], p, g, m, v, None, None) is None   # lr not a number
+    assert h.update(*CALL[:2], torch.tensor(1e-3), *CALL[3:], p, g, m, v, None, None) is None
+    for lr in ("1e-3", None, 10 ** 400):                    # not a number: the per-call path raises
+        assert h.update(*CALL[:2], lr, *CALL[3:], p, g, m, v, None, None) is None
     assert h.update_multi(*CALL, [(p, g, m, v)] * 2, None) is None
     assert h.update_multi(*CALL, [], None) is None
     assert h.update_multi(*CALL, [(p, g, m)], None) is None
