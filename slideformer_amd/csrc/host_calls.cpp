@@ -52,11 +52,36 @@ bool registered(int p, int g, int s)
     return g != LA_BF16 && (s == LA_F32 || (s == LA_F16 && g == LA_F16));
 }
 
-// A plain torch.Tensor or Parameter with memory of its own on HIP device `dev`,
-// contiguous; null otherwise.
+// Whether a tensor answers for itself as torch.Tensor does: a plain tensor or
+// Parameter, or a subclass that leaves __torch_function__ and the methods read
+// here as they are and does not dispatch to Python (such a one has no memory of
+// its own, or hides it).
+bool own_answers(PyObject* o)
+{
+    if (THPVariable_CheckExact(o)) return true;
+    if (!THPVariable_Check(o) || THPVariable_Unpack(o).unsafeGetTensorImpl()->is_python_dispatch()) return false;
+    PyObject* type = reinterpret_cast<PyObject*>(Py_TYPE(o));
+    auto same = [type](PyObject* base, const char* name) {
+        PyObject *a = PyObject_GetAttrString(type, name), *b = PyObject_GetAttrString(base, name);
+        // a class method is bound anew at every look: what it is bound to counts
+        const bool bound = a && b && PyMethod_Check(a) && PyMethod_Check(b);
+        const bool equal = a && b && (bound ? PyMethod_GET_FUNCTION(a) == PyMethod_GET_FUNCTION(b) : a == b);
+        Py_XDECREF(a);
+        Py_XDECREF(b);
+        PyErr_Clear();
+        return equal;
+    };
+    if (!same(THPVariableClass, "__torch_function__") && !same(ParameterClass, "__torch_function__")) return false;
+    for (const char* name : {"data_ptr", "numel", "is_contiguous", "get_device", "dtype", "is_cuda"})
+        if (!same(THPVariableClass, name)) return false;
+    return true;
+}
+
+// A tensor that answers for itself, with memory of its own on HIP device
+// `dev`, contiguous; null otherwise.
 const at::Tensor* plain(PyObject* o, int64_t dev)
 {
-    if (!THPVariable_CheckExact(o)) return nullptr;
+    if (!own_answers(o)) return nullptr;
     const at::Tensor& t = THPVariable_Unpack(o);
     if (!t.defined() || t.layout() != at::kStrided || !t.is_cuda() || t.get_device() != dev || !t.has_storage() ||
         !t.is_contiguous())
@@ -69,7 +94,7 @@ bool coefficient(PyObject* o, int64_t dev, const float** out)
 {
     *out = nullptr;
     if (o == Py_None) return true;
-    if (!THPVariable_CheckExact(o)) return false;
+    if (!own_answers(o)) return false;
     const at::Tensor& t = THPVariable_Unpack(o);
     if (!t.defined() || t.layout() != at::kStrided || !t.is_cuda() || t.get_device() != dev || !t.has_storage() ||
         t.scalar_type() != at::kFloat || t.numel() < 1)

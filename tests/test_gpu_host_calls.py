@@ -29,7 +29,7 @@ def _bits(t):
 
 @pytest.mark.parametrize("form", ["plain", "subclass", "overlap", "mixed grads", "pageable", "pinned", "half on host"])
 def test_step_equals_one_call_per_tensor(form, hip_device):
-    """Plain tensors (batched), a tensor subclass, two tensors that share memory
+    """Plain tensors and a tensor subclass (batched), two tensors that share memory
     and grads of two types (one call each), host tensors (queued, the last one
     waits) and a layer whose second half is on the host."""
     dtype = torch.bfloat16 if form == "plain" else torch.float32
@@ -105,6 +105,40 @@ def test_hyper_parameters_of_any_number_type_keep_the_batched_launch(kind, hip_d
     returned, got = _step(hip_device, *_layer(hip_device, torch.float32, 4), lr=lr, betas=(np.float32(0.9), 0.999))
     assert returned == [0]
     for a, b in zip(got, _step(hip_device, *_layer(hip_device, torch.float32, 4))[1]):
+        assert np.array_equal(a, b)
+
+
+class _Scale(torch.nn.Parameter):
+    pass
+
+
+class _View(torch.Tensor):
+    pass
+
+
+class _Elsewhere(torch.Tensor):
+    """A subclass with an answer of its own."""
+
+    def data_ptr(self):
+        return super().data_ptr()
+
+
+@pytest.mark.parametrize("kind,batched", [("parameter", True), ("grad and clip", True), ("own answer", False)])
+def test_tensor_subclasses_keep_the_batched_launch(kind, batched, hip_device):
+    """Subclasses that leave torch's methods as they are go in one launch, as plain tensors do; one that answers
+    for itself is asked, call by call."""
+    params, grads = _layer(hip_device, torch.float32, 6)
+    coef = torch.tensor([0.5], device=hip_device)
+    if kind == "parameter":
+        params = [_Scale(p.detach()) for p in params]
+    elif kind == "grad and clip":
+        grads, coef = [g.as_subclass(_View) for g in grads], coef.as_subclass(_View)
+    else:
+        grads[1] = grads[1].as_subclass(_Elsewhere)
+    returned, got = _step(hip_device, params, grads, coef)
+    assert returned == [0 if batched else None]
+    plain = _step(hip_device, *_layer(hip_device, torch.float32, 6), torch.tensor([0.5], device=hip_device))[1]
+    for a, b in zip(got, plain):
         assert np.array_equal(a, b)
 
 
