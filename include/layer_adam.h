@@ -28,7 +28,7 @@
 extern "C" {
 #endif
 
-#define LA_ABI_VERSION 9
+#define LA_ABI_VERSION 10
 
 #define LA_OK 0
 #define LA_EINVAL (-22)
@@ -277,6 +277,11 @@ int la_clip_coef(const double* sqnorm, float max_norm, float* coef, float* norm_
  *   arrays go through the HIP runtime's own bounce buffers.  Changing the
  *   attachment settles every queued call first.  No
  *   reference counterpart: the reference updates pageable state on the CPU.
+ * la_pipeline_use_copy_engines: with on != 0 later calls leave host memory to
+ *   the copy engines, whatever kernels could reach; with 0 (as created) they
+ *   choose as said above.  The update of a call in which the kernel reads and
+ *   writes host memory itself holds compute units while the link is busy; by
+ *   copy engines the call takes longer and leaves them to other kernels.
  */
 #define LA_ON_HOST_P 1u
 #define LA_ON_HOST_M 2u
@@ -306,6 +311,7 @@ int la_pipeline_create(uint64_t chunk_elems, int slots, la_pipeline_t** out);
 int la_pipeline_destroy(la_pipeline_t* pl);
 int la_pipeline_sync(la_pipeline_t* pl);
 int la_pipeline_set_host_staging(la_pipeline_t* pl, void* pinned, uint64_t bytes, int threads);
+int la_pipeline_use_copy_engines(la_pipeline_t* pl, int on);
 int la_pipeline_step(la_pipeline_t* pl, const la_scalars_t* sc, int p_dtype, void* p, int g_dtype,
                      const void* g, int s_dtype, void* m, void* v, uint64_t n, uint16_t* out,
                      unsigned on_host, const float* clip_coef, void* workspace,

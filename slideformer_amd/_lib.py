@@ -24,7 +24,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libs
 HOST_CALLS_PATH = os.path.join(os.path.dirname(LIB_PATH), "_host_calls.so")
 
 # LA_ABI_VERSION of include/layer_adam.h that these bindings declare
-ABI_VERSION = 9
+ABI_VERSION = 10
 
 LA_OK = 0
 LA_EINVAL = -22
@@ -65,6 +65,7 @@ EXPORTED = (
     "la_pipeline_destroy",
     "la_pipeline_sync",
     "la_pipeline_set_host_staging",
+    "la_pipeline_use_copy_engines",
     "la_pipeline_step",
     "la_disk_create",
     "la_disk_create_ex",
@@ -181,6 +182,8 @@ def _declare(L):
     L.la_pipeline_sync.restype = i
     L.la_pipeline_set_host_staging.argtypes = [P, P, u64, i]
     L.la_pipeline_set_host_staging.restype = i
+    L.la_pipeline_use_copy_engines.argtypes = [P, i]
+    L.la_pipeline_use_copy_engines.restype = i
     L.la_pipeline_step.argtypes = [P, SP, i, P, i, P, i, P, P, u64, P, ctypes.c_uint, P, P, u64, P, i,
                                    ctypes.POINTER(LaPipelineStats)]
     L.la_pipeline_step.restype = i

@@ -15,8 +15,9 @@
 // ring of twins: host threads copy sub-chunk i in while they copy an earlier
 // one out and the kernel works on those between.
 //
-// Copy-engine path, for pageable arrays without staging and page-locked ones
-// that kernels cannot reach: the call streams the state through HBM in chunks:
+// Copy-engine path, for pageable arrays without staging, page-locked ones that
+// kernels cannot reach and pipelines that ask for it: the call streams the state
+// through HBM in chunks:
 //
 //   h2d stream :  copy the host-resident arrays among p, m, v, g of chunk i into
 //                 slot i % S
@@ -103,9 +104,6 @@ using la_host::Piece;
 #ifndef LA_DIRECT_SLOTS
 #define LA_DIRECT_SLOTS 6
 #endif
-#ifndef LA_DIRECT
-#define LA_DIRECT 1  // 0: every call takes the copy-engine path
-#endif
 #ifndef LA_DIRECT_LAUNCH
 #define LA_DIRECT_LAUNCH (64ull << 20)
 #endif
@@ -125,6 +123,7 @@ struct la_pipeline {
     char* host_staging = nullptr;
     uint64_t host_staging_bytes = 0;
     bool host_staging_direct = false;  // kernels reach all of it
+    bool copy_engines = false;         // asked for: no call takes the direct path
     std::unique_ptr<CopyPool> pool;
     // the slot ring across calls: whose slots it holds (the copy-engine path's,
     // done at ev_d2h, or the direct path's, done at ev_direct) and how many;
@@ -558,6 +557,13 @@ int la_pipeline_set_host_staging(la_pipeline_t* pl, void* pinned, uint64_t bytes
     return LA_OK;
 }
 
+int la_pipeline_use_copy_engines(la_pipeline_t* pl, int on)
+{
+    if (!pl) return LA_EINVAL;
+    pl->copy_engines = on != 0;  // the ring's change of hands settles what is queued
+    return LA_OK;
+}
+
 int la_pipeline_step(la_pipeline_t* pl, const la_scalars_t* sc, int p_dtype, void* p, int g_dtype, const void* g,
                      int s_dtype, void* m, void* v, uint64_t n, uint16_t* out, unsigned on_host,
                      const float* clip_coef, void* workspace, uint64_t workspace_bytes, la_stream_t after,
@@ -660,7 +666,7 @@ try {
                              {vp, sb, hv, st_v, true, true},
                              {const_cast<char*>(gp), gb, hg, st_g, true, false},
                              {op, 2, ho, st_o, false, true}};
-    bool direct = LA_DIRECT != 0 && (!staged || pl->host_staging_direct);
+    bool direct = !pl->copy_engines && (!staged || pl->host_staging_direct);
     for (const Array& a : arrays)
         if (a.host && !a.staged)
             direct = direct && !misaligned(a.base, a.bytes) &&

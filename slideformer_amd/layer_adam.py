@@ -81,7 +81,7 @@ class HostStreamer:
     arrays to the HIP runtime's own bounce buffers instead."""
 
     def __init__(self, device, chunk_elems: int = HOST_STAGE_ELEMS, slots: int = HOST_STAGE_SLOTS, *,
-                 host_threads: int = 0, stage_pageable: bool = True):
+                 host_threads: int = 0, stage_pageable: bool = True, copy_engines: bool = False):
         self.lib = _lib.load()
         self.device = torch.device(device)
         self.chunk = chunk_elems
@@ -93,6 +93,8 @@ class HostStreamer:
             _lib.check(self.lib.la_pipeline_create(chunk_elems, slots, ctypes.byref(handle)),
                        "la_pipeline_create")
         self.handle = handle
+        if copy_engines:
+            _lib.check(self.lib.la_pipeline_use_copy_engines(handle, 1), "la_pipeline_use_copy_engines")
         self._ws = {}
         self._host_ws = {}
         # every tensor of a call that returned once queued, until the pipeline
@@ -285,6 +287,7 @@ class LayerAdam:
             moments_hbm_bytes: Optional[int] = None,
             stream_chunk_elems: int = HOST_STAGE_ELEMS,
             stream_slots: int = HOST_STAGE_SLOTS,
+            copy_engines: bool = False,
     ):
         """Arguments of the reference (layer_adam.py:17-30), plus keyword-only:
         ``device``: the HIP device that updates host-resident state (default: current);
@@ -316,7 +319,15 @@ class LayerAdam:
         every measured layout but one: a page-locked master with the moments in
         HBM in one call of a very large layer (1.8 B params), where 64 Mi x 3
         runs 150 ms against 180-207 ms (64 MB copies back to the host then go
-        partly to a DMA engine that the other direction also uses)."""
+        partly to a DMA engine that the other direction also uses);
+        ``copy_engines``: leave host-resident arrays to the copy engines.  Without
+        it the update kernel reads and writes them over the link, which is faster
+        but holds compute units while it runs.  A Llama-3.1-8B layer queued with
+        ``overlap_host_chunks``, page-locked, then 24 / 72 bf16 products of 8192^3
+        (19 / 56 ms alone) on the caller's stream, until both are done: 56 / 87 ms,
+        by copy engines 64 / 65; with the moments in HBM 28 / 67 and 27 / 60; the
+        step alone 55 against 64 and 23 against 27.  So it pays where other work
+        fills more of the GPU's time than the step does."""
         self.defaults = dict(
             lr=lr,
             bias_correction=bias_correction,
@@ -359,6 +370,7 @@ class LayerAdam:
         self.moments_hbm_bytes = moments_hbm_bytes
         self.stream_chunk_elems = int(stream_chunk_elems)
         self.stream_slots = int(stream_slots)
+        self.copy_engines = bool(copy_engines)
         self.moments_hbm_used = 0     # bytes of moments placed on moments_device so far
         self.state: DefaultDict[torch.Tensor, Any] = defaultdict(dict)
 
@@ -635,7 +647,8 @@ class LayerAdam:
             streamer = self._streamers.get(device)
             if streamer is None:
                 streamer = self._streamers[device] = HostStreamer(device, chunk_elems=self.stream_chunk_elems,
-                                                                  slots=self.stream_slots)
+                                                                  slots=self.stream_slots,
+                                                                  copy_engines=self.copy_engines)
             on_host = _placement(params, grads, exp_avg, exp_avg_sq, bf16_out)
             self.last_stream_stats = streamer.step(
                 sc, pc, params, gc, grads, sc_, exp_avg, exp_avg_sq, n, bf16_out, on_host,

@@ -352,13 +352,16 @@ struct Run {
 
 // Calls that wait and calls that return once queued, in random order on the
 // parts of a layer: what a waiting call or a sync leaves is the reference's.
-static void results(const Layout& l, uint64_t n, int slots, int threads)
+// `engines`: by copy engines; `turns`: asked for them now and then.
+static void results(const Layout& l, uint64_t n, int slots, int threads, bool engines, bool turns)
 {
     Run r(l, n, slots, threads);
+    CHECK(la_pipeline_use_copy_engines(r.pl, engines ? 1 : 0) == LA_OK);
     std::mt19937 rng(static_cast<unsigned>(n) * 31u + static_cast<unsigned>(slots));
     g_copies = g_updates = g_links = 0;
     for (int call = 0; call < 24; ++call) {
         const bool wait = rng() % 4 == 0;
+        if (turns && rng() % 3 == 0) CHECK(la_pipeline_use_copy_engines(r.pl, static_cast<int>(rng() % 2)) == LA_OK);
         CHECK(r.step(rng() % kParts, wait) == LA_OK);
         if (wait) {
             CHECK(work_queued() == 0);
@@ -369,15 +372,18 @@ static void results(const Layout& l, uint64_t n, int slots, int threads)
     run_all(&g_null);
     CHECK(work_queued() == 0);
     CHECK(r.same());
-    CHECK(l.direct ? g_links > 0 && g_updates == 0 && g_copies == 0 : g_links == 0 && g_updates > 0 && g_copies > 0);
+    const bool direct = l.direct && !engines;
+    CHECK(turns || (direct ? g_links > 0 && g_updates == 0 && g_copies == 0
+                           : g_links == 0 && g_updates > 0 && g_copies > 0));
 }
 
 // Every submission of a call fails in turn: once the call has returned its
 // error, nothing that it or an earlier call queued reads or writes memory any more.
-static void failures(const Layout& l, uint64_t n, int slots, bool wait, bool behind_others)
+static void failures(const Layout& l, uint64_t n, int slots, bool wait, bool behind_others, bool engines)
 {
     for (int k = 0;; ++k) {
         Run r(l, n, slots, 2);
+        CHECK(la_pipeline_use_copy_engines(r.pl, engines) == LA_OK);
         if (behind_others) CHECK(r.step(0, false) == LA_OK && r.step(1, false) == LA_OK);
         g_submitted = 0;
         g_fail_at = k;
@@ -393,6 +399,7 @@ static void failures(const Layout& l, uint64_t n, int slots, bool wait, bool beh
 
 int main()
 {
+    CHECK(la_pipeline_use_copy_engines(nullptr, 1) == LA_EINVAL);
     for (const bool lazy : {true, false}) {
         g_lazy = lazy;
         for (const Layout& l : kLayouts)
@@ -401,7 +408,9 @@ int main()
                     std::printf("%s, %llu elements, %d slots, %s\n", l.name, static_cast<unsigned long long>(n), slots,
                                 lazy ? "late" : "at once");
                     std::fflush(stdout);
-                    results(l, n, slots, 1 + slots);
+                    results(l, n, slots, 1 + slots, false, false);
+                    results(l, n, slots, 1 + slots, true, false);
+                    results(l, n, slots, 1 + slots, false, true);
                 }
     }
     g_lazy = true;
@@ -409,8 +418,10 @@ int main()
         for (const bool wait : {true, false}) {
             std::printf("%s, failing, %s\n", l.name, wait ? "waiting" : "queued");
             std::fflush(stdout);
-            failures(l, 3000, 2, wait, false);
-            failures(l, 1000, 2, wait, true);
+            for (const bool engines : {false, true}) {
+                failures(l, 3000, 2, wait, false, engines);
+                failures(l, 1000, 2, wait, true, engines);
+            }
         }
     std::printf("pipeline driver ok\n");
     return 0;
