@@ -162,3 +162,43 @@ def test_queued_calls_of_every_route_on_one_pipeline(hip_device):
                 assert np.array_equal(H.to_np_bits(t, "f32"), x[lo:hi].view(np.uint32)), (step, kind)
     del parts, p, m, v, t, adam, streamer, coarse
     _lib._hip().hipHostFree(owner)
+
+
+@pytest.mark.parametrize("triple,offsets", [
+    (("bf16", "bf16", "f32"), (1, 3, 2, 1, 5)),      # odd elements, no head aligns all: the misphased form
+    (("bf16", "bf16", "bf16"), (1, 2, 5, 7, 3)),
+    (("f16", "f16", "f16"), (3, 3, 3, 3, 3)),        # one odd phase for all: a head of 5
+    (("f16", "f32", "f32"), (1, 0, 1, 3, 0)),
+    (("f32", "bf16", "f32"), (1, 3, 0, 2, 7)),
+])
+@pytest.mark.parametrize("n", [1, 31, 4097, 100_003])
+def test_page_locked_arrays_at_odd_elements(triple, offsets, n, hip_device):
+    """Host arrays of every element size that start at odd elements, which the kernel reads and writes over the link
+    in place, the host's bf16 copy included; what lies beside them stays as it is.  Bit-exact with the checker."""
+    rng = np.random.default_rng(n + offsets[0])
+    kinds = (triple[0], triple[1], triple[2], triple[2], "bf16")
+    k16 = [None if k == "f32" else k for k in triple]
+    values = [rng.normal(0, 0.02, n), None, rng.normal(0, 1e-3, n), np.abs(rng.normal(0, 1e-5, n)), np.zeros(n)]
+    pads, arrays = [], []
+    for x, kind, off in zip(values, kinds, offsets):
+        pad = torch.full((off + n + 9,), 7.0, dtype=H.TD[kind]).pin_memory()
+        pads.append((pad, off))
+        arrays.append(pad[off:off + n])
+        if x is not None:
+            arrays[-1].copy_(torch.from_numpy(x.astype(np.float32)).to(H.TD[kind]))
+    p, g, m, v, out = arrays
+    ref = [H.to_np_bits(t, k) for t, k in zip(arrays, kinds)]
+    view = lambda b, k: b.view(np.float32) if k == "f32" else b
+    adam = streamed(hip_device, chunk_elems=16384, slots=2)
+    orc = O.OracleAdam(1e-3, (0.9, 0.999), 1e-8, 0.01, True)
+    for step in (1, 2, 3):
+        print(f"odd elements {triple} {offsets} n={n} step={step}", flush=True)
+        g.copy_(torch.from_numpy(rng.normal(0, 1e-3, n).astype(np.float32)).to(g.dtype))
+        adam.step_chunk(p, g, m, v, dict(adam.defaults, step=step), bf16_out=out)
+        assert direct(adam.last_stream_stats)
+        orc.update(step, *HP, view(ref[0], kinds[0]), view(H.to_np_bits(g, kinds[1]), kinds[1]), view(ref[2], kinds[2]),
+                   view(ref[3], kinds[3]), p16=k16[0], g16=k16[1], s16=k16[2], p_bf16_out=ref[4])
+        for j in (0, 2, 3, 4):
+            assert np.array_equal(H.to_np_bits(arrays[j], kinds[j]), ref[j]), (step, j)
+    for pad, off in pads:
+        assert (pad[:off] == 7.0).all() and (pad[off + n:] == 7.0).all()
