@@ -49,15 +49,16 @@ def test_check_grads_names_the_first_refused_grad():
         h.check_grads([None], 0)
 
 
-def test_a_host_tensor_is_refused_without_a_device_and_the_scalars_have_advanced():
-    if torch.cuda.is_available():
-        pytest.skip("needs a machine without a HIP device")
+def test_a_host_tensor_is_refused_without_a_device_and_the_scalars_stay(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: False)
     adam = LayerAdam(lr=1e-3)
     adam.add_layer_params(0, [torch.nn.Parameter(_cpu()), torch.nn.Parameter(_cpu())])
     for q in adam.param_groups[0]["params"]:
         q.grad = _cpu()
     with pytest.raises(RuntimeError, match="HIP device"):
         adam.step(0)
+    sc = adam._scalars(1, 1e-3, 0.9, 0.999, 1e-8, 0.0, True)     # the first call that advances the powers of beta
+    assert sc.step == 1 and sc.beta1_t == sc.beta1 and sc.beta2_t == sc.beta2
 
 
 @pytest.mark.parametrize("overlap", [False, True])
