@@ -150,12 +150,23 @@
 // The copy engines move 48 GB/s each way at once, 57 one way alone.  An 8192^3
 // bf16 product beside it takes 1.5 ms (0.83 alone) with 32 x 256, 1.37 with
 // 16 x 512 and 2.3-2.5 with workgroups on all 256 compute units.
+// Where a wave reads few bytes over the link per trip, 128 waves leave it idle
+// between: 56 GB/s need ~100 KB of host reads in flight, whatever the wave
+// reads from HBM beside them.  So a call whose waves read at most 512 bytes of
+// host memory per trip (2-byte grads or parameters beside fp32 moments) takes
+// twice the workgroups.  Measured, 218 M elements, ms per call, 32 / 48 / 64 / 96
+// workgroups, and by copy engines: grads on the host 11.0 / 8.0 / 7.7 / 7.6, 8.2;
+// grads and bf16 copy 11.9 / 8.9 / 8.7 / 9.7, 9.7; bf16 parameters 11.8 / 8.9 /
+// 8.7 / 9.6, 9.7.  At 1 KB per trip and more, or none read, more workgroups are
+// no faster: fp32 parameters 17.4 / 19.2 / 18.3 / 17.6, 18.9, grads of all-16-bit
+// triples 7.8 / 7.7 / 7.6 / 8.4, 8.2, the copy alone 8.0 / 7.8 / 8.1 / 7.9, 8.1.
 #ifndef LA_LINK_BLOCK
 #define LA_LINK_BLOCK 256
 #endif
 #ifndef LA_LINK_GRID
 #define LA_LINK_GRID 32
 #endif
+constexpr unsigned kLinkFewBytes = 512;
 static_assert(LA_BLOCK % 64 == 0 && LA_LINK_BLOCK % 64 == 0, "workgroups are whole waves");
 static_assert(static_cast<unsigned long long>(LA_MAX_GRID) * LA_BLOCK <= 0xffffffffull,
               "the grid size in work-items must fit the dispatch packet's 32 bits");
@@ -842,13 +853,15 @@ template <typename TP, typename TG, typename TS> struct StepLauncher {
 
 // The same kernel on host memory (see LA_LINK_GRID).
 template <typename TP, typename TG, typename TS> struct LinkLauncher {
-    static int run(const StepArgs& a, hipStream_t stream)
+    static int run(const StepArgs& a, unsigned link_read, hipStream_t stream)
     {
         const uint64_t nscalar = a.head + (a.n - (a.head + a.nvec * lane_elems<TP, TG, TS>()));
         const uint64_t work = a.nvec > nscalar ? a.nvec : nscalar;
+        const unsigned wave_reads = link_read * 64 * lane_elems<TP, TG, TS>();
+        const uint64_t grid = wave_reads > 0 && wave_reads <= kLinkFewBytes ? 2 * LA_LINK_GRID : LA_LINK_GRID;
         return launch(a.misphased ? la_adamw_kernel<TP, TG, TS, true, LA_LINK_BLOCK>
                                   : la_adamw_kernel<TP, TG, TS, false, LA_LINK_BLOCK>,
-                      dim3(grid_for(work, LA_LINK_BLOCK, LA_LINK_GRID)), dim3(LA_LINK_BLOCK), 0, stream, a);
+                      dim3(grid_for(work, LA_LINK_BLOCK, grid)), dim3(LA_LINK_BLOCK), 0, stream, a);
     }
 };
 
@@ -1145,13 +1158,13 @@ int scratch_on_current_device(int dev, double** out)
 namespace la_link {
 
 int step(const la_scalars_t& sc, int p_dtype, void* p, int g_dtype, const void* g, int s_dtype, void* m, void* v,
-         uint64_t n, uint16_t* p_bf16_out, const float* clip_coef, hipStream_t stream)
+         uint64_t n, uint16_t* p_bf16_out, const float* clip_coef, unsigned link_read, hipStream_t stream)
 {
     StepArgs a;
     const int rc = prepare_step(p_dtype, p, g_dtype, g, s_dtype, m, v, n, p_bf16_out, clip_coef, a, true);
     if (rc != LA_OK) return rc;
     set_coeffs(sc, a.k);
-    return dispatch_triple<LinkLauncher>(p_dtype, g_dtype, s_dtype, a, stream);
+    return dispatch_triple<LinkLauncher>(p_dtype, g_dtype, s_dtype, a, link_read, stream);
 }
 
 }  // namespace la_link

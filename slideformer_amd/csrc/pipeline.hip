@@ -319,8 +319,10 @@ int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtyp
     const bool wait = synchronize || stats;
     bool staged = false;
     for (int k = 0; k < kArrays; ++k) staged |= a[k].staged;
+    unsigned link_read = 0;
     uint64_t h2d_bytes = 0, d2h_bytes = 0, staged_bytes = 0;
     for (int k = 0; k < kArrays; ++k) {
+        if (a[k].host && a[k].in) link_read += static_cast<unsigned>(a[k].bytes);
         if (a[k].host && a[k].in) h2d_bytes += n * a[k].bytes;
         if (a[k].host && a[k].out) d2h_bytes += n * a[k].bytes;
     }
@@ -393,7 +395,7 @@ int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtyp
         for (int j = 0; j < kArrays; ++j)
             at[j] = a[j].staged ? twin + region[j] : a[j].base ? a[j].base + off * a[j].bytes : nullptr;
         const int rc = la_link::step(sc, p_dtype, at[0], g_dtype, at[3], s_dtype, at[1], at[2], k,
-                                     reinterpret_cast<uint16_t*>(at[4]), clip_coef, st);
+                                     reinterpret_cast<uint16_t*>(at[4]), clip_coef, link_read, st);
         if (rc != LA_OK) return drain_streams(pl, rc);
         if (staged) {
             LA_DIRECT_TRY(hipEventRecord(pl->ev_direct[s], st));

@@ -230,9 +230,13 @@ extern "C" int la_adamw_step(const la_scalars_t*, int, void* p, int, const void*
 }
 namespace la_link {
 int step(const la_scalars_t&, int, void* p, int, const void* g, int, void* m, void* v, uint64_t n, uint16_t* out,
-         const float*, hipStream_t st)
+         const float*, unsigned link_read, hipStream_t st)
 {
     ++g_links;
+    unsigned host = 0;   // what it reads of host memory
+    for (const void* x : {static_cast<const void*>(p), g, static_cast<const void*>(m), static_cast<const void*>(v)})
+        host += region(x)->device ? 0u : 4u;
+    CHECK(link_read == host);
     return launch(p, g, m, v, n, out, st, true);
 }
 }  // namespace la_link

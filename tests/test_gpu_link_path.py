@@ -202,3 +202,34 @@ def test_page_locked_arrays_at_odd_elements(triple, offsets, n, hip_device):
             assert np.array_equal(H.to_np_bits(arrays[j], kinds[j]), ref[j]), (step, j)
     for pad, off in pads:
         assert (pad[:off] == 7.0).all() and (pad[off + n:] == 7.0).all()
+
+
+# around one trip of 32 and of 64 workgroups, and several
+@pytest.mark.parametrize("n", [5, 32_768, 32_785, 65_536, 65_551, 200_003])
+@pytest.mark.parametrize("triple,host", [(("f32", "bf16", "f32"), "g"), (("bf16", "bf16", "f32"), "p"),
+                                         (("f16", "f16", "f32"), "go"), (("bf16", "bf16", "bf16"), "g")])
+def test_calls_that_read_few_bytes_over_the_link(triple, host, n, hip_device):
+    """Only the grads or 16-bit parameters (and the bf16 copy) in page-locked memory, the rest in HBM: the launch
+    shape for waves that read at most 512 bytes of host memory per trip, and the all-16-bit triple, which reads more.
+    Bit-exact with the checker."""
+    rng = np.random.default_rng(n)
+    kinds = dict(p=triple[0], g=triple[1], m=triple[2], v=triple[2], o="bf16")
+    scale = dict(p=0.02, m=1e-3, v=1e-5, o=0.0)
+    place = lambda t, name: t.pin_memory() if name in host else t.to(hip_device)
+    make = lambda s, k: torch.from_numpy(rng.normal(0, 1, n).astype(np.float32) * np.float32(s)).to(H.TD[k])
+    t = {k: place(make(scale[k], kinds[k]).abs() if k == "v" else make(scale[k], kinds[k]), k) for k in "pmvo"}
+    ref = {k: H.to_np_bits(t[k], kinds[k]) for k in "pmvo"}
+    k16 = {k: None if x == "f32" else x for k, x in kinds.items()}
+    view = lambda b, k: b.view(np.float32) if k == "f32" else b
+    adam = streamed(hip_device, chunk_elems=16384, slots=2)
+    orc = O.OracleAdam(1e-3, (0.9, 0.999), 1e-8, 0.01, True)
+    for step in (1, 2):
+        print(f"few bytes over the link {triple} {host} n={n} step={step}", flush=True)
+        g = make(1e-3, kinds["g"])
+        adam.step_chunk(t["p"], place(g, "g"), t["m"], t["v"], dict(adam.defaults, step=step), bf16_out=t["o"])
+        assert direct(adam.last_stream_stats)
+        orc.update(step, *HP, view(ref["p"], kinds["p"]), view(H.to_np_bits(g, kinds["g"]), kinds["g"]),
+                   view(ref["m"], kinds["m"]), view(ref["v"], kinds["v"]), p16=k16["p"], g16=k16["g"], s16=k16["m"],
+                   p_bf16_out=ref["o"])
+        for k in "pmvo":
+            assert np.array_equal(H.to_np_bits(t[k], kinds[k]), ref[k]), (step, k)
