@@ -92,6 +92,16 @@ using la_host::Piece;
 // 496 / 1500.  A Llama-3.1-8B layer in 32 Mi calls: copy engines 97.1 ms,
 // direct 64.4; within 3 % with sub-chunks of 0.5-4 Mi and 4-10 twins, bound by
 // the host's memory (the threads' and the device's traffic share it).
+// Those are the bounds for LA_DIRECT_STAGED bytes per element through the
+// threads, both ways together; with fewer staged they are as many times larger,
+// so that a round still copies enough to pay for waking the threads.  Up to four
+// copies of the size that the calling thread makes alone the smaller bound stays.
+// Pageable grads alone / bf16 copy alone / bf16 master, state in HBM, ms per call
+// with elements for bounds, with bytes, by copy engines: 3 M elements 0.41 / 0.39
+// / 0.57, 0.25 / 0.24 / 0.30, 0.28 / 0.29 / 0.48; 218 M 12.6 / 10.5 / 13.7, 8.2 /
+// 8.2 / 9.6, 8.5 / 8.3 / 10.3 (from 9.4 / 9.5 / 11.5 with the launch's wider grid
+// alone).  6, 12 and 36 bytes: 3 M 0.26 / 0.25 / 0.60, 0.24 / 0.24 / 0.44, 0.25 /
+// 0.25 / 0.53, and 218 M within 2 % of 24 but for the master with 6 (11.4).
 // Page-locked arrays: a launch of 64 Mi runs ~17 ms, and other work on the
 // device gets a gap between launches.  Same layer, master page-locked, moments
 // in HBM: copy engines 26.8 ms, direct 23.3 (56 GB/s in).
@@ -100,6 +110,9 @@ using la_host::Piece;
 #endif
 #ifndef LA_DIRECT_SUB_MIN
 #define LA_DIRECT_SUB_MIN (1ull << 18)
+#endif
+#ifndef LA_DIRECT_STAGED
+#define LA_DIRECT_STAGED 24
 #endif
 #ifndef LA_DIRECT_SLOTS
 #define LA_DIRECT_SLOTS 6
@@ -300,6 +313,28 @@ uint64_t direct_layout(uint64_t sub, const Array* a, uint64_t* region)
     return off;
 }
 
+// Bytes per element that the host threads copy into the twins and out of them.
+struct StagedBytes {
+    uint64_t in = 0, out = 0;
+    // how many times LA_DIRECT_SUB and LA_DIRECT_SUB_MIN elements bound a sub-chunk
+    uint64_t scale() const { return std::max<uint64_t>(1, LA_DIRECT_STAGED / (in + out)); }
+};
+StagedBytes staged_per_element(const Array* a)
+{
+    StagedBytes s;
+    for (int k = 0; k < kArrays; ++k) {
+        if (a[k].staged && a[k].in) s.in += static_cast<uint64_t>(a[k].bytes);
+        if (a[k].staged && a[k].out) s.out += static_cast<uint64_t>(a[k].bytes);
+    }
+    return s;
+}
+
+// Most elements of a sub-chunk, of a call with staged arrays.
+uint64_t direct_sub(const la_pipeline* pl, const Array* a)
+{
+    return std::min<uint64_t>(pl->chunk, LA_DIRECT_SUB * staged_per_element(a).scale());
+}
+
 // The ring of a direct call.  A call without staged arrays uses no slots; it
 // leaves the ring of earlier direct calls as it is, since it only adds to the
 // one stream that they share.
@@ -307,7 +342,7 @@ int enter_direct(la_pipeline* pl, const Array* a, bool staged)
 {
     if (!staged) return pl->ring_direct || pl->ring_slots == 0 ? LA_OK : enter_ring(pl, true, 0, nullptr, 0);
     uint64_t region[kArrays];
-    const uint64_t slot = direct_layout(std::min<uint64_t>(pl->chunk, LA_DIRECT_SUB), a, region);
+    const uint64_t slot = direct_layout(direct_sub(pl, a), a, region);
     // the staging holds at least `slots` slots of `chunk` elements of every host array
     return enter_ring(pl, true, std::min<uint64_t>(LA_DIRECT_SLOTS, pl->host_staging_bytes / slot), pl->host_staging,
                       slot);
@@ -368,9 +403,12 @@ int direct_step(la_pipeline* pl, const la_scalars_t& sc, int p_dtype, int g_dtyp
     uint64_t region[kArrays] = {};
     const uint64_t S = pl->ring_slots;
     if (staged) {
-        const uint64_t sub = std::min<uint64_t>(pl->chunk, LA_DIRECT_SUB);
+        const uint64_t sub = direct_sub(pl, a);
         (void)direct_layout(sub, a, region);
-        step = std::min(sub, std::max<uint64_t>(LA_DIRECT_SUB_MIN, round_up(n / 8, 16)));
+        const StagedBytes per = staged_per_element(a);
+        // few bytes in all: sub-chunks that the calling thread copies alone are the quicker ones
+        const bool alone = n * std::max(per.in, per.out) <= 4 * la_host::kAloneBytes;
+        step = std::min(sub, std::max<uint64_t>(LA_DIRECT_SUB_MIN * (alone ? 1 : per.scale()), round_up(n / 8, 16)));
     }
     for (uint64_t off = 0; off < n; off += step) {
         const uint64_t k = std::min(step, n - off);

@@ -401,8 +401,25 @@ static void failures(const Layout& l, uint64_t n, int slots, bool wait, bool beh
     }
 }
 
+// Sub-chunks of staged arrays: an eighth of the call, at least so many elements
+// that a round of the host threads copies enough, unless there is little in all.
+// The build's bounds are 32 and 128 elements of 24 staged bytes, kAloneBytes 1024.
+static int sub_chunks(const Layout& l, uint64_t n)
+{
+    Run r(l, n, 2, 2);
+    g_links = 0;
+    CHECK(r.step(0, true) == LA_OK && r.same());
+    return g_links;
+}
+
 int main()
 {
+    const Layout grads = {"pageable grads", kDevice, kDevice, kPageable, kDevice, true, true};
+    const Layout state = {"pageable state", kPageable, kPageable, kDevice, kDevice, true, true};
+    CHECK(sub_chunks(state, 1100) == 9);    // 24 bytes an element: most 128
+    CHECK(sub_chunks(grads, 1000) == 8);    // 4 bytes, 4000 in all: eighths
+    CHECK(sub_chunks(grads, 1100) == 6);    // 4 bytes: at least 6 x 32
+    CHECK(sub_chunks(grads, 5000) == 20);   // and at most 6 x 128, here the chunk's 256
     CHECK(la_pipeline_use_copy_engines(nullptr, 1) == LA_EINVAL);
     for (const bool lazy : {true, false}) {
         g_lazy = lazy;
