@@ -596,12 +596,24 @@ constexpr uint32_t kBeyond = 1u << 30;  // an offset outside every run's descrip
 // of 4099 elements 8.2 against 15.6, the 9 of a layer of hidden size 2048 (54 M)
 // 22.1 against 26.0, of 4096 (218 M, whole trips of the walk) 71.3 against 70.0;
 // one buffer of 7.1 M 6.5 against 7.0, of 218 M 69.4 against 68.9.
+// A trip that meets a buffer's end takes ~0.25 us more than one inside a buffer,
+// which the other waves' loads hide as long as all waves take as many of them.
+// So after its trips inside a buffer a wave takes the general trip at once, also
+// where the next buffer starts with that trip: waves beside it may have to.  Only
+// where every buffer is whole trips, and no wave ever has to, all trips are the
+// plain ones (`whole`).  clip_grad_norm, us, the walk / general trips / this
+// rule / plain trips wherever they fit: 32 buffers of 4 Mi 44.2 / 52.2 / 44.0 /
+// 44.0, 32 of 8 Mi 86.0 / 91.4 / 86.2 / 86.4, 32 of 4 Mi + 13 61.9 / 54.6 / 54.4
+// / 55.1, the 9 of hidden size 4096 71.2 / 72.3 / 72.3 / 73.5.
 template <int N> struct NormBuffers {
     // buffer count - 1 - j of the call at index j
     const void* g[N];
     uint64_t n[N], head[N], nvec[N];
+    const void* top[N];   // the end of its aligned groups
     uint32_t run_end[N];  // runs of buffers 0 .. j
+    uint32_t last[N];     // groups of its last run
     int32_t count;
+    int32_t whole;        // every buffer is whole trips of the grid
     NormArgs end;         // where the sum goes
 };
 
@@ -615,20 +627,18 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N>
     const int count = N == 1 ? 1 : a.count;
     const uint32_t runs = a.run_end[count - 1];
     double acc = 0.0;
-    // the buffer of the run at hand: its runs [begin, end), its first aligned
-    // group, the groups of its last run, its end
+    // the buffer of the run at hand: its runs [begin, end), the groups of its last
+    // run, its end
     int b = -1;
     uint32_t begin = 0, end = 0, last = 0;
-    const TG *bottom = nullptr, *top = nullptr;
+    const TG* top = nullptr;
     auto seek = [&](uint32_t r) {
         while (r >= end && b + 1 < count) {
             ++b;
             begin = end;
             end = a.run_end[b];
-            const uint64_t nvec = a.nvec[b];
-            bottom = static_cast<const TG*>(a.g[b]) + a.head[b];
-            top = bottom + nvec * kVec;
-            last = (static_cast<uint32_t>(nvec) - 1) % 64 + 1;
+            last = a.last[b];
+            top = static_cast<const TG*>(a.top[b]);
         }
     };
     auto add = [&acc](const Raw4<TG>& raw) {
@@ -643,8 +653,9 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N>
     for (uint32_t r0 = w; r0 < runs;) {
         seek(r0);
         Raw4<TG> raw[LA_NORM_UNROLL];
-        // trips inside one buffer, before its last run, which may be partial
-        for (; r0 + (LA_NORM_UNROLL - 1) * waves + 1 < end; r0 += LA_NORM_UNROLL * waves) {
+        // trips inside one buffer, of 64 groups in every run
+        const uint32_t full = last == 64 ? end : end - 1;
+        for (; r0 + (LA_NORM_UNROLL - 1) * waves < full; r0 += LA_NORM_UNROLL * waves) {
             const TG* at = top - (static_cast<uint64_t>(r0 - begin) * 64 + lane + 1) * kVec;
 #pragma unroll
             for (int u = 0; u < LA_NORM_UNROLL; ++u)
@@ -652,7 +663,7 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N>
 #pragma unroll
             for (int u = 0; u < LA_NORM_UNROLL; ++u) add(raw[u]);
         }
-        if (r0 >= runs) break;
+        if (r0 >= (a.whole ? end : runs)) continue;
         // a trip that meets a buffer's end: every load through the descriptor of
         // its own run, empty past the last run; lane l takes the l-th group from
         // the run's top, or none (an offset beyond the descriptor)
@@ -661,7 +672,7 @@ __global__ __launch_bounds__(LA_NORM_BLOCK) void la_sqnorm_kernel(NormBuffers<N>
             const uint32_t r = r0 + u * waves;
             seek(r);
             const uint32_t groups = r + 1 < end ? 64u : r < end ? last : 0u;
-            const TG* lo = groups == 64 ? top - (static_cast<uint64_t>(r - begin) + 1) * (64 * kVec) : bottom;
+            const TG* lo = top - (static_cast<uint64_t>(r - begin) * 64 + groups) * kVec;
             raw[u].template load<NT ? kAux : 0>(
                 WaveIo<TG>::rsrc(lo, 0, groups * kVec),
                 lane < groups ? (groups - 1 - lane) * static_cast<uint32_t>(kVec * sizeof(TG)) : kBeyond);
@@ -1019,6 +1030,8 @@ int launch_sqnorm(int g_dtype, const la_grad_buffer_t* bufs, int count, uint32_t
     m.count = count;
     m.end = end;
     const int gb = elem_bytes(g_dtype);
+    const uint64_t trip = static_cast<uint64_t>(grid) * LA_NORM_BLOCK * LA_NORM_UNROLL;  // groups
+    m.whole = 1;
     uint32_t runs = 0;
     for (int j = 0; j < count; ++j) {
         const la_grad_buffer_t& q = bufs[count - 1 - j];
@@ -1032,6 +1045,9 @@ int launch_sqnorm(int g_dtype, const la_grad_buffer_t* bufs, int count, uint32_t
         }
         runs += static_cast<uint32_t>((m.nvec[j] + 63) / 64);
         m.run_end[j] = runs;
+        m.last[j] = m.nvec[j] ? static_cast<uint32_t>((m.nvec[j] - 1) % 64 + 1) : 0;
+        m.top[j] = static_cast<const char*>(q.g) + (m.head[j] + m.nvec[j] * kVec) * static_cast<uint64_t>(gb);
+        if (m.nvec[j] % trip) m.whole = 0;
     }
     // plain loads for the read that produces the coefficient, nontemporal otherwise
     const bool nt = !(end.coef && LA_NORM_CLIP_PLAIN);

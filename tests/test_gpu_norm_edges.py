@@ -203,3 +203,27 @@ def test_sqnorm_is_the_running_sum_itself(hip_device):
     c_ref, n_ref = O.clip_coef(held.item(), 0.25)
     assert abs(held.item() - 9.0 * want) <= 9e-12 * want
     assert coef.item() == np.float32(c_ref) and norm.item() == np.float32(n_ref)
+
+
+TRIP = 32_768     # elements that the small-grid build's two workgroups read in one trip
+
+
+@pytest.mark.parametrize("kind", ["bf16", "f32", "f16"])
+@pytest.mark.parametrize("sizes,off", [((TRIP, TRIP), 0), ((2 * TRIP, 0, TRIP, 3 * TRIP, 0), 0), ((0, TRIP), 0),
+                                       ((TRIP, TRIP - 256, TRIP), 0), ((TRIP + 256, TRIP), 0),
+                                       ((TRIP + 4, TRIP - 4), 0), ((3 * TRIP + 3, 2 * TRIP + 1), 1)])
+def test_norm_over_buffers_of_whole_trips(sizes, off, kind, hip_device):
+    """Buffers that are whole trips of the grid, alone, with empty ones among them, and beside one whose last run or
+    last trip is not whole; also whole but for the elements before and after the aligned groups."""
+    L = H.load_small_grid()
+    bufs = [(torch.randn(n + 8, device=hip_device) * 1e-2).to(H.TD[kind])[off:off + n] for n in sizes]
+    exact = sum(O.grad_sqnorm(_bits(g, kind), None if kind == "f32" else kind) for g in bufs if g.numel())
+    for order in (bufs, bufs[::-1]):
+        ws = torch.full((2,), float("nan"), dtype=torch.float64, device=hip_device)
+        sq = torch.full((1,), float("nan"), dtype=torch.float64, device=hip_device)
+        flat = [x for g in order for x in (g.data_ptr(), g.numel())]
+        arr = ctypes.cast((ctypes.c_uint64 * len(flat))(*flat), ctypes.POINTER(_lib.LaGradBuffer))
+        print(f"whole trips {sizes} {off} {kind}", flush=True)
+        assert L.la_grad_norm_multi(H.CODE[kind], arr, len(order), ws.data_ptr(), 16, sq.data_ptr(), 0, 0.0, None,
+                                    None, torch.cuda.current_stream().cuda_stream) == 0
+        assert abs(sq.item() - exact) <= 1e-12 * exact
