@@ -95,7 +95,6 @@ __device__ __forceinline__ uint32_t f32_to_f16_bits(float f)
     return __builtin_bit_cast(uint16_t, static_cast<_Float16>(f));
 }
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <typename V, bool NT = (LA_NT_LOAD != 0)> __device__ __forceinline__ V vload(const void* p)
@@ -113,21 +112,10 @@ template <typename V> __device__ __forceinline__ void vstore(void* p, V v)
 #endif
 }
 
-// 4 consecutive elements <-> 4 floats; `e` is a multiple of 4 past an aligned head.
+// Element `e` of a stream, alone.
 template <typename T> struct Io;
 
 template <> struct Io<float> {
-    static constexpr int kBytes = 4;
-    template <bool NT = (LA_NT_LOAD != 0)>
-    __device__ __forceinline__ static void load4(const void* base, uint64_t e, float (&x)[kVec])
-    {
-        const f32x4 a = vload<f32x4, NT>(static_cast<const float*>(base) + e);
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
-    }
-    __device__ __forceinline__ static void store4(void* base, uint64_t e, const float (&x)[kVec])
-    {
-        vstore<f32x4>(static_cast<float*>(base) + e, f32x4{x[0], x[1], x[2], x[3]});
-    }
     __device__ __forceinline__ static float load1(const void* base, uint64_t e)
     {
         return static_cast<const float*>(base)[e];
@@ -139,22 +127,6 @@ template <> struct Io<float> {
 };
 
 template <typename Conv> struct Io16 {
-    static constexpr int kBytes = 2;
-    template <bool NT = (LA_NT_LOAD != 0)>
-    __device__ __forceinline__ static void load4(const void* base, uint64_t e, float (&x)[kVec])
-    {
-        const u32x2 u = vload<u32x2, NT>(static_cast<const uint16_t*>(base) + e);
-        x[0] = Conv::to_f32(u.x & 0xffffu);
-        x[1] = Conv::to_f32(u.x >> 16);
-        x[2] = Conv::to_f32(u.y & 0xffffu);
-        x[3] = Conv::to_f32(u.y >> 16);
-    }
-    __device__ __forceinline__ static void store4(void* base, uint64_t e, const float (&x)[kVec])
-    {
-        const uint32_t lo = Conv::from_f32x2(x[0], x[1]);
-        const uint32_t hi = Conv::from_f32x2(x[2], x[3]);
-        vstore<u32x2>(static_cast<uint16_t*>(base) + e, u32x2{lo, hi});
-    }
     __device__ __forceinline__ static float load1(const void* base, uint64_t e)
     {
         return Conv::to_f32(static_cast<const uint16_t*>(base)[e]);
