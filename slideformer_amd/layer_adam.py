@@ -10,14 +10,16 @@ the same methods (``add_layer_params``, ``step``, ``step_with_grad_views``,
 beta-power state machine of the reference runs on the host inside that library.
 
 Device tensors are updated in place, asynchronously on the current HIP stream.
-Host tensors (the reference's layout: fp32 master and moments in CPU RAM) are
-streamed through HBM in 16 Mi-element chunks by the library's native
-three-stream pipeline (H2D / update / D2H overlapped) and the call returns
-after completion, as the reference's CPU call does.  Each array of a call may
-be on the host or on the one device; only the host-resident ones cross the
-host link (``LayerAdam(moments_device=...)`` keeps the moments in HBM beside a
-host-resident master).  Pageable host arrays are copied through page-locked
-staging by native host threads.  There is no CPU arithmetic path.
+Host tensors (the reference's layout: fp32 master and moments in CPU RAM) go
+through the library's native pipeline, and the call returns after completion, as
+the reference's CPU call does.  The update kernel reads and writes page-locked
+arrays over the host link; pageable ones are copied through page-locked staging
+by native host threads, a part at a time; arrays that kernels cannot reach, and
+all of them where ``copy_engines`` asks for it, stream through HBM in chunks.
+Each array of a call may be on the host or on the one device; only the
+host-resident ones cross the host link (``LayerAdam(moments_device=...)`` keeps
+the moments in HBM beside a host-resident master).  There is no CPU arithmetic
+path.
 
 Additions, all keyword-only so that positional signatures are unchanged:
 ``bf16_out=`` (the bf16 compute copy written in the same pass), ``clip_coef=``
@@ -56,11 +58,12 @@ SUPPORTED_TRIPLES = frozenset({
     (torch.float32, torch.float16, torch.float32),
 })
 
-# Host tensors are streamed through HBM in chunks of this many elements (64 MB
-# of fp32 per state array), through HOST_STAGE_SLOTS staging slots.  A multiple
-# of 16, so that only the last chunk of a call holds the reference's scalar
-# tail (the last n % 16 elements of the call).  Measured on MI355X over one
-# Llama-3.1-8B layer: with page-locked state, 4-16 Mi-element chunks with 3-4
+# Where the copy engines move host tensors, they stream them through HBM in
+# chunks of this many elements (64 MB of fp32 per state array), through
+# HOST_STAGE_SLOTS staging slots; the staging of pageable arrays has that size on
+# either path.  A multiple of 16, so that only the last chunk of a call holds the
+# reference's scalar tail (the last n % 16 elements of the call).  Measured on
+# MI355X over one Llama-3.1-8B layer, by copy engines: with page-locked state, 4-16 Mi-element chunks with 3-4
 # slots all run at 46-47.5 GB/s each way (the concurrent-duplex limit of the
 # host link); with pageable state staged by host threads, 16 Mi x 3 runs at
 # 59-60 ms per layer every time, while with four slots a D2H hipMemcpyAsync
@@ -75,10 +78,11 @@ class HostStreamer:
     device staging memory it needs (allocated here, never by the library).
 
     Pageable host arrays (the reference's moments are plain ``torch.zeros``,
-    layer_adam.py:161-173) go through page-locked twins of the staging slots,
-    copied by ``host_threads`` native threads (0 = up to 16); the copy engines
-    then only see page-locked memory.  ``stage_pageable=False`` leaves pageable
-    arrays to the HIP runtime's own bounce buffers instead."""
+    layer_adam.py:161-173) go through page-locked twins, copied by
+    ``host_threads`` native threads (0 = up to 16); the device then only sees
+    page-locked memory.  ``stage_pageable=False`` leaves pageable arrays to the
+    HIP runtime's own bounce buffers instead; ``copy_engines`` as in
+    ``LayerAdam``."""
 
     def __init__(self, device, chunk_elems: int = HOST_STAGE_ELEMS, slots: int = HOST_STAGE_SLOTS, *,
                  host_threads: int = 0, stage_pageable: bool = True, copy_engines: bool = False):
@@ -314,7 +318,9 @@ class LayerAdam:
         temporary the caller drops is not freed early;
         ``stream_chunk_elems``, ``stream_slots``: the chunk (elements, rounded
         down to a multiple of 16) and the number of device staging slots with
-        which host-resident arrays stream through HBM.  The defaults, 16 Mi
+        which the copy engines stream host-resident arrays through HBM, and the
+        size of the staging for pageable ones.  Page-locked arrays that kernels
+        reach do not depend on them.  By copy engines the defaults, 16 Mi
         elements (64 MB of fp32) and 3 slots, are the best or near it for
         every measured layout but one: a page-locked master with the moments in
         HBM in one call of a very large layer (1.8 B params), where 64 Mi x 3
@@ -451,8 +457,8 @@ class LayerAdam:
             **self.defaults,
         }
         self.param_groups.append(param_group)
-        # host moments are page-locked on request: the copy engines then read and
-        # write them directly, without the staging copies that pageable arrays
+        # host moments are page-locked on request: the device then reads and
+        # writes them directly, without the staging copies that pageable arrays
         # take (not with the file offload, which releases and re-allocates them);
         # at their exact size, since a process may page-lock only so much
         pin = (device.type == 'cpu' and self.pin_host_state and self.offloader is None
@@ -814,7 +820,7 @@ class LayerAdam:
         convention), one-element views of this call's scratch.  Pass ``coef`` as
         ``clip_coef=`` to ``step_chunk``.  The grads go to the library in runs of
         one dtype, up to 32 tensors per la_grad_norm_multi call (two launches
-        each).  Nothing is synchronised with the host.
+        each, one up to 131,072 elements).  Nothing is synchronised with the host.
         """
         grads = [g for g in grads if g is not None]
         if not grads:
@@ -884,7 +890,8 @@ class GradNormAccumulator:
 
     def add(self, grad, *, stream=None) -> None:
         """Add one grad buffer, or a sequence of them (a layer's per-tensor
-        grads: two launches for up to 32 tensors of one dtype)."""
+        grads: two launches for up to 32 tensors of one dtype, one up to 131,072
+        elements)."""
         grads = [grad] if isinstance(grad, torch.Tensor) else [g for g in grad if g is not None]
         if not grads:
             return
