@@ -125,6 +125,7 @@ def _calls(test):
     "test_moments_hbm_budget_splits_layers",
     "test_pipeline_other_triples_staged_and_overlapped",
     "test_async_pipeline_calls_with_changing_layouts",
+    "test_c5_streamed_full_size_matches_resident",
     "test_pipeline_equals_resident_on_random_layouts",
 ])
 def test_pipeline_tests_on_the_copy_engines(name, hip_device, monkeypatch):
