@@ -272,13 +272,14 @@ def _hip():
         return _hip_runtime
 
 
-# start address -> bytes of every live page_locked_empty allocation
+# start address -> bytes of every live page_locked_empty allocation.  Without a
+# lock: each use is one dict operation, and the garbage collector may run
+# _release in a thread that holds a lock or walks the table.
 _page_locked = {}
 
 
 def _release(rt, address: int) -> None:
-    with _lock:
-        _page_locked.pop(address, None)
+    _page_locked.pop(address, None)
     rt.hipHostFree(address)
 
 
@@ -291,8 +292,7 @@ def is_page_locked(t: torch.Tensor) -> bool:
     if t.is_pinned():
         return True
     ptr = t.data_ptr()
-    with _lock:
-        return any(start <= ptr < start + size for start, size in _page_locked.items())
+    return any(start <= ptr < start + size for start, size in _page_locked.copy().items())
 
 
 def page_locked_empty(numel: int, dtype: torch.dtype) -> torch.Tensor:
@@ -314,8 +314,7 @@ def page_locked_empty(numel: int, dtype: torch.dtype) -> torch.Tensor:
     if rc != 0 or not ptr.value:
         raise RuntimeError(f"hipHostMalloc of {nbytes} bytes failed (hipError_t {rc})")
     raw = np.frombuffer((ctypes.c_uint8 * max(1, nbytes)).from_address(ptr.value), dtype=np.uint8)
-    with _lock:
-        _page_locked[ptr.value] = max(1, nbytes)
+    _page_locked[ptr.value] = max(1, nbytes)
     # Not at interpreter exit: finalizers then run in no fixed order, possibly
     # before a pipeline that still copies into this memory has been drained;
     # the process's own teardown reclaims it.

@@ -15,7 +15,7 @@ loader instead::
 ``adam_update`` routes by where the four tensors live:
 
 * all four in host memory (what the reference's ``step`` / ``step_chunk``
-  pass, ``layer_adam.py:314-327,448-461``): streamed through HBM by the native
+  pass, ``layer_adam.py:314-327,448-461``): the native
   chunk pipeline (``la_pipeline_step``) on the current HIP device; the call
   returns after completion, as the reference's CPU call does;
 * all four on one HIP device: one ``la_adam_update`` launch, asynchronous on
@@ -136,7 +136,7 @@ def adam_update(optimizer_id, step, lr, beta1, beta2, epsilon, weight_decay, bia
 
 
 def _host_step(L, sc, codes, tensors, n):
-    """Host-resident p, g, m, v: streamed through HBM on the current HIP device
+    """Host-resident p, g, m, v: the native pipeline on the current HIP device
     (every placement bit set), complete on return."""
     from .layer_adam import HostStreamer
     device = torch.device("cuda", torch.cuda.current_device())

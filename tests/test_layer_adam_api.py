@@ -255,6 +255,44 @@ def test_offload_cleanup_leaves_other_processes_files(tmp_path):
     assert foreign.read_bytes() == b"another run's moments"
 
 
+def test_a_page_locked_finalizer_needs_no_lock():
+    """The garbage collector runs finalizers in whatever thread allocates, also one that holds the module's lock
+    (the native host module is loaded under it) or walks the table: the finalizer of a page-locked allocation must
+    not wait for either."""
+    import threading
+
+    from slideformer_amd import _lib
+
+    class Runtime:
+        freed = []
+
+        def hipHostFree(self, address):
+            self.freed.append(address)
+
+    def finalize_under_the_lock():
+        with _lib._lock:
+            _lib._release(Runtime(), 4096)
+
+    _lib._page_locked[4096] = 64
+    t = threading.Thread(target=finalize_under_the_lock, daemon=True)
+    t.start()
+    t.join(10)
+    assert not t.is_alive() and Runtime.freed == [4096] and 4096 not in _lib._page_locked
+
+    class Walked(int):
+        """An address whose comparison finalizes an allocation, as a collection during the walk would."""
+
+        def __le__(self, other):
+            _lib._release(Runtime(), 8192)
+            return int(self) <= other
+
+    _lib._page_locked.update({Walked(1): 1, 8192: 64})
+    try:
+        assert not _lib.is_page_locked(torch.zeros(4))
+    finally:
+        _lib._page_locked.pop(1, None)
+
+
 def test_is_page_locked_of_plain_host_memory():
     from slideformer_amd import _lib
     assert not _lib.is_page_locked(torch.zeros(16))
